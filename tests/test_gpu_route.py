@@ -96,6 +96,51 @@ def test_group_router(gpu, oracle, T, E, k, ng, tg, in_dtype, out_dtype):
         _check_rows(inds.cpu().numpy(), _w_np(w), oi, ow, key, wtol)
 
 
+@pytest.mark.parametrize("T,E,k,ng,tg", [
+    (6, 1, 1, 0, 0),        # one expert
+    (6, 63, 63, 0, 0),      # every expert picked, one lane idle
+    (5, 65, 10, 0, 0),      # one expert past a whole wave
+    (4, 1024, 64, 0, 0),    # the largest row
+    (5, 96, 9, 3, 2),       # group counts that are no power of two
+    (5, 130, 12, 5, 3),
+    (3, 1024, 8, 2, 1),     # the longest groups: 32 lanes each
+    (7, 64, 64, 64, 64),    # one lane per group, every expert picked
+])
+def test_router_ties(gpu, oracle, T, E, k, ng, tg):
+    """Rows of few distinct values: equal scores go to the lower index, inside a lane's
+    slots, across lanes and across groups.  Values 1/4 apart are far from any rounding,
+    so the picks equal the oracle's exactly."""
+    from fastmlx_amd import ops
+
+    announce(f"router ties T={T} E={E} k={k} groups={ng}/{tg}")
+    g = torch.Generator().manual_seed(E + k)
+    x = torch.randint(-3, 4, (T, E), generator=g).float() * 0.25
+    if ng:
+        inds, w = ops.route_group_topk(x.to(gpu), None, k, ng, tg, 1.0, True)
+        oi, ow = oracle.route_group_topk(x.numpy(), np.zeros(E, np.float32), k, ng, tg, 1.0, True)
+    else:
+        inds, w = ops.route_softmax_topk(x.to(gpu), k, True, torch.float32)
+        oi, ow = oracle.route_softmax_topk(x.numpy(), k, norm=True)
+    torch.cuda.synchronize()
+    assert np.array_equal(inds.cpu().numpy(), oi)
+    assert np.allclose(_w_np(w), ow, rtol=1e-5, atol=1e-7)
+
+
+def test_router_masked_experts(gpu):
+    """A correction bias of -inf takes an expert out; with fewer finite scores than
+    picks the masked ones follow in index order, and a NaN score is never picked."""
+    from fastmlx_amd import ops
+
+    announce("router with -inf biases and a NaN")
+    x = torch.zeros(1, 70)
+    x[0, 3], x[0, 69], x[0, 40] = 2.0, 1.0, float("nan")
+    bias = torch.full((70,), float("-inf"))
+    bias[3] = bias[69] = bias[40] = 0.0
+    inds, _ = ops.route_group_topk(x.to(gpu), bias.to(gpu), 4, 1, 1, 1.0, True)
+    torch.cuda.synchronize()
+    assert inds[0].cpu().tolist() == [3, 69, 0, 1]
+
+
 def test_group_router_reference_vectors(gpu):
     """The reference fixture of TestDeepseekV3GroupExpertSelectParity
     (compute/models/deepseekv3_test.go:130-163) through the HIP router."""
