@@ -509,7 +509,7 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
   uint32_t* flag = nullptr;
   if (int rc = device_flag(static_cast<hipStream_t>(stream), &flag)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (Mx == 1 && E <= kSortMaxExperts && fmxq::moe_qmvs_supported(N, K, bits, group_size) &&
+  if (Mx == 1 && E <= kSortMaxExperts && fmxq::moe_qmvs_supported(N, K, x_batch, bits, group_size) &&
       aligned16(scales) && aligned16(biases)) {
     // Items sorted by expert, then one grouped product per expert segment; the
     // sort's order maps each sorted item back to its output row.
@@ -517,7 +517,7 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
       // A few items: each is its own segment, written to its own output row.
       fmxq::MoeArgs a{x, lhs_indices, {w, nullptr}, {scales, nullptr}, {biases, nullptr},
                       rhs_indices, nullptr, nullptr, y, nullptr, batch, N, K, E, x_batch, flag,
-                      lhs_div};
+                      group_size, bits, lhs_div};
       return hip_status(fmxq::launch_moe_qmvs(a, 1, 16, batch, s), op);
     }
     const int window = fmxq::moe_window(batch, E);
@@ -536,7 +536,7 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
                               "gather_qmm: sort"))
         return rc;
       fmxq::MoeArgs a{x, m.lhs, {w, nullptr}, {scales, nullptr}, {biases, nullptr}, m.rhs,
-                      m.seg, m.nseg, y, m.order, batch, N, K, E, x_batch, flag};
+                      m.seg, m.nseg, y, m.order, batch, N, K, E, x_batch, flag, group_size, bits};
       if (int rc = hip_status(fmxq::launch_moe_qmvs(a, 1, window, max_seg, s), op)) return rc;
       if (!max_tiles) return FMXQ_OK;
       const fmxq::QmmArgs gq = grouped_args(x, w, scales, biases, y, N, K, bits, group_size, m,
@@ -620,8 +620,8 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
   const int window = fmxq::moe_window(S, E);
   const int64_t max_seg = fmxq::moe_max_segments(S, E, window);
   if (E <= kSortMaxExperts && max_seg <= kMaxSegmentsGrid &&
-      fmxq::moe_qmvs_supported(I, D, bits, group_size) &&
-      fmxq::moe_qmvs_supported(D, I, bits, group_size) && aligned16(s_gate) &&
+      fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
+      fmxq::moe_qmvs_supported(D, I, S + T, bits, group_size) && aligned16(s_gate) &&
       aligned16(b_gate) && aligned16(s_up) && aligned16(b_up) && aligned16(s_down) &&
       aligned16(b_down)) {
     // Sorted slots (for every slot count: the order cannot change a value, each
@@ -632,11 +632,11 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
     if (S <= fmxq::kMoeUnsortedMaxSlots) {
       if (int rc = moe_scratch(s, S, I, 1, &m, op, 0, 0, src)) return rc;
       fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
-                       nullptr, m.h, nullptr, S, I, D, E, T, flag, topk};
+                       nullptr, m.h, nullptr, S, I, D, E, T, flag, group_size, bits, topk};
       if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, 16, S, s), "switch_glu: gate/up"))
         return rc;
       fmxq::MoeArgs dn{m.h, nullptr, {w_down, nullptr}, {s_down, nullptr}, {b_down, nullptr},
-                       inds, nullptr, nullptr, out, nullptr, S, D, I, E, S, flag, 1};
+                       inds, nullptr, nullptr, out, nullptr, S, D, I, E, S, flag, group_size, bits, 1};
       return hip_status(fmxq::launch_moe_qmvs(dn, 1, 16, S, s), "switch_glu: down");
     }
     // Long expert runs (>= kGroupedMinRun slots) go to the grouped GEMM: gate and
@@ -655,7 +655,7 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
                             "switch_glu: sort"))
       return rc;
     fmxq::MoeArgs gu{x, m.lhs, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, m.rhs, m.seg,
-                     m.nseg, m.h, nullptr, S, I, D, E, T, flag};
+                     m.nseg, m.h, nullptr, S, I, D, E, T, flag, group_size, bits};
     if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, window, max_seg, s),
                             "switch_glu: gate/up"))
       return rc;
@@ -675,7 +675,7 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
         return rc;
     }
     fmxq::MoeArgs dn{m.h, nullptr, {w_down, nullptr}, {s_down, nullptr}, {b_down, nullptr},
-                     m.rhs, m.seg, m.nseg, out, m.order, S, D, I, E, S, flag};
+                     m.rhs, m.seg, m.nseg, out, m.order, S, D, I, E, S, flag, group_size, bits};
     if (int rc = hip_status(fmxq::launch_moe_qmvs(dn, 1, window, max_seg, s), "switch_glu: down"))
       return rc;
     if (!max_tiles) return FMXQ_OK;
@@ -777,19 +777,19 @@ extern "C" int fmxq_switch_glu_combine(
   // up into h (no sort), then one kernel for the down projection and the combine.
   if (fmxq::moe_combine_unsorted(S, E) &&
       fmxq::moe_down_combine_supported(T, topk, D, I, bits, group_size) &&
-      fmxq::moe_qmvs_supported(I, D, bits, group_size) && aligned16(s_gate) &&
+      fmxq::moe_qmvs_supported(I, D, T, bits, group_size) && aligned16(s_gate) &&
       aligned16(b_gate) && aligned16(s_up) && aligned16(b_up)) {
     uint32_t* flag = nullptr;
     if (int rc = device_flag(static_cast<hipStream_t>(stream), &flag)) return rc;
     MoeScratch m;
     if (int rc = moe_scratch(s, S, I, 1, &m, op)) return rc;
     fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
-                     nullptr, m.h, nullptr, S, I, D, E, T, flag, topk};
+                     nullptr, m.h, nullptr, S, I, D, E, T, flag, group_size, bits, topk};
     if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, 16, S, s), "switch_glu_combine: gate/up"))
       return rc;
     return hip_status(fmxq::launch_moe_down_combine(m.h, inds, w_down, s_down, b_down, weights,
                                                     shared, shared_gate, out, T, topk, E, D, I,
-                                                    flag, s),
+                                                    group_size, bits, flag, s),
                       "switch_glu_combine: down/combine");
   }
   // Otherwise the two calls in sequence, the expert rows in the arena's slot 1.
@@ -834,7 +834,7 @@ extern "C" int fmxq_moe_layer(
   // and one more wave of each down/combine block, two launches for the layer.
   if (T == 1 && topk <= 15 && fmxq::moe_combine_unsorted(S, E) && D >= 2048 && D <= 16384 &&
       fmxq::moe_down_combine_supported(T, topk, D, I, bits, group_size) &&
-      fmxq::moe_qmvs_supported(I, D, bits, group_size) && aligned16(s_gate) &&
+      fmxq::moe_qmvs_supported(I, D, T, bits, group_size) && aligned16(s_gate) &&
       aligned16(b_gate) && aligned16(s_up) && aligned16(b_up) && aligned16(ss_gate) &&
       aligned16(sb_gate) && aligned16(ss_up) && aligned16(sb_up)) {
     uint32_t* flag = nullptr;
@@ -842,7 +842,7 @@ extern "C" int fmxq_moe_layer(
     MoeScratch m;
     if (int rc = moe_scratch(s, S + T, I, 1, &m, op)) return rc;
     fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
-                     nullptr, m.h, nullptr, S, I, D, E, T, flag, topk};
+                     nullptr, m.h, nullptr, S, I, D, E, T, flag, group_size, bits, topk};
     gu.sh_w[0] = sw_gate;
     gu.sh_w[1] = sw_up;
     gu.sh_s[0] = ss_gate;
@@ -854,7 +854,7 @@ extern "C" int fmxq_moe_layer(
       return rc;
     return hip_status(fmxq::launch_moe_down_combine(m.h, inds, w_down, s_down, b_down, weights,
                                                     nullptr, shared_gate, out, T, topk, E, D, I,
-                                                    flag, s, sw_down, ss_down, sb_down),
+                                                    group_size, bits, flag, s, sw_down, ss_down, sb_down),
                       "moe_layer: down/combine");
   }
   // Sorted batches below the grouped GEMM's floor: the shared expert joins the
@@ -867,8 +867,8 @@ extern "C" int fmxq_moe_layer(
     const int64_t max_seg = fmxq::moe_max_segments(Sa, E + 1, window);
     if (!fmxq::moe_combine_unsorted(S, E) && grouped_max_tiles(S, E) == 0 &&
         E + 1 <= kSortMaxExperts && max_seg <= kMaxSegmentsGrid &&
-        fmxq::moe_qmvs_supported(I, D, bits, group_size) &&
-        fmxq::moe_qmvs_supported(D, I, bits, group_size) && aligned16(s_gate) &&
+        fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
+        fmxq::moe_qmvs_supported(D, I, S + T, bits, group_size) && aligned16(s_gate) &&
         aligned16(b_gate) && aligned16(s_up) && aligned16(b_up) && aligned16(s_down) &&
         aligned16(b_down) && aligned16(ss_gate) && aligned16(sb_gate) && aligned16(ss_up) &&
         aligned16(sb_up) && aligned16(ss_down) && aligned16(sb_down)) {
@@ -886,7 +886,7 @@ extern "C" int fmxq_moe_layer(
                               "moe_layer: sort"))
         return rc;
       fmxq::MoeArgs gu{x, m.lhs, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, m.rhs, m.seg,
-                       m.nseg, m.h, nullptr, Sa, I, D, E, T, flag};
+                       m.nseg, m.h, nullptr, Sa, I, D, E, T, flag, group_size, bits};
       gu.sh_w[0] = sw_gate;
       gu.sh_w[1] = sw_up;
       gu.sh_s[0] = ss_gate;
@@ -898,7 +898,7 @@ extern "C" int fmxq_moe_layer(
                               "moe_layer: gate/up"))
         return rc;
       fmxq::MoeArgs dn{m.h, nullptr, {w_down, nullptr}, {s_down, nullptr}, {b_down, nullptr},
-                       m.rhs, m.seg, m.nseg, y, m.order, Sa, D, I, E, Sa, flag};
+                       m.rhs, m.seg, m.nseg, y, m.order, Sa, D, I, E, Sa, flag, group_size, bits};
       dn.sh_w[0] = sw_down;
       dn.sh_s[0] = ss_down;
       dn.sh_b[0] = sb_down;

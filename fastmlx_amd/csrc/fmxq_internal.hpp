@@ -240,8 +240,8 @@ hipError_t launch_quantize(const uint16_t* w, uint32_t* wq, uint16_t* scales, ui
                            int64_t rows, int64_t K, int group_size, int bits,
                            hipStream_t stream);
 
-// Grouped int4 (group 64, K a multiple of 256) product over expert segments of
-// a sorted slot order (fmxq_moe_gemm.hip).  w/s/b hold NMAT stacks [E, N, .]
+// Grouped product (4 or 8 bits, groups of 32, 64 or 128, K a multiple of 256) over
+// expert segments of a sorted slot order (fmxq_moe_gemm.hip).  w/s/b hold NMAT stacks [E, N, .]
 // (gate and up for NMAT = 2, which writes silu(gate) * up); slot s reads x row
 // lhs ? lhs[s] : s and writes output row yrow ? yrow[s] : s.
 struct MoeArgs {
@@ -257,6 +257,7 @@ struct MoeArgs {
   const uint32_t* yrow;     // [S] or null
   int64_t S, N, K, E, x_rows;
   uint32_t* err_flag;
+  int group_size, bits;
   int64_t lhs_div = 1;      // x row of slot s is lhs[s], or s / lhs_div without lhs
   // Few-slot GEMV form only (no segment table, no yrow): sh_T more segments after
   // the S slots, segment S + t the shared expert (sh_w / sh_s / sh_b, one [N, .]
@@ -283,11 +284,17 @@ constexpr int64_t kMoeUnsortedCombineMaxSlots = 256;
 inline bool moe_combine_unsorted(int64_t S, int64_t E) {
   return S <= kMoeUnsortedMaxSlots || (S <= kMoeUnsortedCombineMaxSlots && 2 * S <= E);
 }
-bool moe_qmvs_supported(int64_t N, int64_t K, int bits, int group_size);
+bool moe_qmvs_supported(int64_t N, int64_t K, int64_t x_rows, int bits, int group_size);
 int moe_window(int64_t S, int64_t E);
 int64_t moe_max_segments(int64_t S, int64_t E, int window);
 hipError_t launch_moe_qmvs(const MoeArgs& a, int nmat, int window, int64_t max_seg,
                            hipStream_t stream);
+// The shared-x walk for the formats other than 4 bits in groups of 64
+// (fmxq_moe_walk_q4.hip, fmxq_moe_walk_q8.hip).
+hipError_t launch_moe_qmvw_q4(const MoeArgs& a, int nmat, int window, int ntt, int64_t max_seg,
+                              hipStream_t stream);
+hipError_t launch_moe_qmvw_q8(const MoeArgs& a, int nmat, int window, int ntt, int64_t max_seg,
+                              hipStream_t stream);
 
 // Few-slot down projection fused with the top-k combine (one block per row
 // tile and token, one wave per slot): out [T, D] from the h rows [T k, I].
@@ -301,8 +308,8 @@ hipError_t launch_moe_down_combine(const uint16_t* h, const uint32_t* inds, cons
                                    const uint16_t* s, const uint16_t* b, const uint16_t* weights,
                                    const uint16_t* shared, const uint16_t* sgate, uint16_t* out,
                                    int64_t T, int64_t k, int64_t E, int64_t D, int64_t I,
-                                   uint32_t* err_flag, hipStream_t stream,
-                                   const uint32_t* sh_w = nullptr, const uint16_t* sh_s = nullptr,
+                                   int group_size, int bits, uint32_t* err_flag,
+                                   hipStream_t stream, const uint32_t* sh_w = nullptr, const uint16_t* sh_s = nullptr,
                                    const uint16_t* sh_b = nullptr);
 // Fill n uint32 words with v (a kernel, so it can sit in a captured graph).
 hipError_t launch_fill_u32(uint32_t* p, uint32_t v, int64_t n, hipStream_t stream);

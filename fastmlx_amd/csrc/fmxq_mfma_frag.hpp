@@ -88,6 +88,14 @@ __device__ __forceinline__ bf16x8 deq_frag8(uint32_t w0, uint32_t w1, float s, f
   return __builtin_bit_cast(bf16x8, r);
 }
 
+// Two 8-bit words as bf16(q) in natural order: integers up to 255 are exact in bf16.
+__device__ __forceinline__ bf16x8 cvt_frag8(uint32_t w0, uint32_t w1) {
+  return as_bf16x8(pack_bf16x2((float)(w0 & 0xffu), (float)((w0 >> 8) & 0xffu)),
+                   pack_bf16x2((float)((w0 >> 16) & 0xffu), (float)(w0 >> 24)),
+                   pack_bf16x2((float)(w1 & 0xffu), (float)((w1 >> 8) & 0xffu)),
+                   pack_bf16x2((float)((w1 >> 16) & 0xffu), (float)(w1 >> 24)));
+}
+
 // Exponent-trick offset per value and the factor that turns the ones-MFMA sum of
 // the A operand back into sum x (int8 A carries every x value twice).
 template <int BITS>

@@ -77,15 +77,190 @@ __device__ __forceinline__ f32x4 qmvs_bias4(float xs, float bo, f32x4 acc) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(xs, bo, acc, 0, 0, 0);
 }
 
-template <int NTT, int SU, int BITS = 4>
+// Exact B operand of one MFMA: one int4 word as bf16(128 + q) in pair order, or two
+// int8 words as bf16(q) in natural order.
+template <int BITS>
+__device__ __forceinline__ bf16x8 qmvs_bfrag(const uint32_t* w) {
+  if constexpr (BITS == 4) return wfrag<4>(w[0]);
+  else return cvt_frag8(w[0], w[1]);
+}
+
+template <int NTT, int SU, int BITS = 4, int GS = 64>
 struct QmvsGeom {
   static constexpr int ROWS = 16 * NTT;
   static constexpr int RB = SU * 8 * BITS;     // bytes of one row per step
   static constexpr int LPR = RB / 16;          // lanes per row in one load instruction
   static constexpr int NI = ROWS * RB / 1024;  // load instructions per step
-  static constexpr int SPL = (64 / ROWS == 2) ? SU : SU / 2;  // groups per scale load
+  static constexpr int GPS = SU * 64 / GS;     // quantization groups per step
+  // Scale loads of one step: 16-row tiles have lanes to spare, so two lanes share a
+  // row's groups (unless a step has only two, which each of them then loads).
+  static constexpr int HALVES = (ROWS == 16 && GPS >= 4) ? 2 : 1;
+  static constexpr int SPL = GPS / HALVES;     // groups per scale load
   static constexpr int STAGE = ROWS * RB;      // LDS bytes per matrix
 };
+
+// Order of K inside a 64-value unit.  Each MFMA of a unit takes 32 of its values, 8
+// per lane quarter q.  Groups of 64 and more: quarter q holds the 16 consecutive
+// values from 16 q (one LDS read), MFMA h its 8 values h.  Groups of 32: MFMA h
+// must stay inside group h, so quarter q holds values 32 h + 8 q .. + 8.
+// x chunk (16 bytes, 8 values) of unit j for MFMA h:
+template <int GS>
+__device__ __forceinline__ int qmvs_xchunk(int j, int h, int q) {
+  return GS == 32 ? 8 * j + 4 * h + q : 8 * j + 2 * q + h;
+}
+
+// The packed words of one unit as this lane's B operands: BITS / 4 words for MFMA 0,
+// then as many for MFMA 1, read from row r of a stage (row base `row`, chunks at
+// qmvs_pos).  off0 / off1 are the byte offsets from the row base (qmvs_woff).
+template <int BITS, int GS>
+struct QmvsWords {
+  uint32_t v[BITS / 2];
+};
+template <int BITS, int GS, int RB>
+__device__ __forceinline__ int qmvs_woff(int j, int h, int q, int r) {
+  if constexpr (BITS == 8) {
+    if constexpr (GS == 32) return (qmvs_pos<RB / 32>(4 * j + 2 * h + (q >> 1), r) << 4) + (q & 1) * 8;
+    else return qmvs_pos<RB / 32>(4 * j + q, r) << 4;
+  } else {
+    if constexpr (GS == 32) return (qmvs_pos<RB / 32>(2 * j + h, r) << 4) + q * 4;
+    else return (qmvs_pos<RB / 32>(2 * j + (q >> 1), r) << 4) + (q & 1) * 8;
+  }
+}
+template <int BITS, int GS>
+__device__ __forceinline__ QmvsWords<BITS, GS> qmvs_read_words(const uint8_t* stage, int off0,
+                                                               int off1) {
+  QmvsWords<BITS, GS> w;
+  if constexpr (GS == 32 && BITS == 4) {
+    w.v[0] = *reinterpret_cast<const uint32_t*>(stage + off0);
+    w.v[1] = *reinterpret_cast<const uint32_t*>(stage + off1);
+  } else if constexpr (GS == 32) {
+    const u32x2 a = *reinterpret_cast<const u32x2*>(stage + off0);
+    const u32x2 b = *reinterpret_cast<const u32x2*>(stage + off1);
+    w.v[0] = a[0], w.v[1] = a[1], w.v[2] = b[0], w.v[3] = b[1];
+  } else if constexpr (BITS == 4) {
+    const u32x2 a = *reinterpret_cast<const u32x2*>(stage + off0);
+    w.v[0] = a[0], w.v[1] = a[1];
+  } else {
+    const u32x4 a = *reinterpret_cast<const u32x4*>(stage + off0);
+    w.v[0] = a[0], w.v[1] = a[1], w.v[2] = a[2], w.v[3] = a[3];
+  }
+  return w;
+}
+
+// The MFMAs of one step: acc += x . w over the step's SU units.  load_a(mt, j, h)
+// returns the x chunk of tile mt for MFMA h of unit j; sv / bv hold the step's scale
+// and bias pairs (groups 2k, 2k + 1).
+//   DEQ: the weights dequantized, w = bf16(fma(s, q, b)).
+//   otherwise the exact affine form per group: P = sum x (OFF + q), xs = sum x (an
+//   MFMA against ones), acc += s P + (b - OFF s) xs, with OFF = 128 and exponent-trick
+//   operands for 4 bits, OFF = 0 and q itself (exact in bf16) for 8; with FOLD the
+//   second term of four groups goes in as one fp32 MFMA.
+template <int MTW, int MT, int NTT, int NMAT, int SU, bool FOLD, bool DEQ, int BITS, int GS, class LoadA>
+__device__ __forceinline__ void qmvs_step_mma(
+    LoadA&& load_a, const QmvsWords<BITS, GS> (&wv)[SU][NMAT][NTT],
+    const uint32_t (&sv)[NMAT][NTT][SU * 32 / GS], const uint32_t (&bv)[NMAT][NTT][SU * 32 / GS],
+    f32x4 (&acc)[NMAT][MT][NTT]) {
+  static_assert(!(DEQ && FOLD), "DEQ accumulates the dequantized product directly");
+  constexpr int GM = GS / 32;         // MFMAs per group
+  constexpr int GPS = SU * 64 / GS;   // groups per step
+  constexpr float OFF = BITS == 4 ? 128.f : 0.f;
+  auto scale = [&](int p, int t, int g) { return (g & 1) ? bf16_hi(sv[p][t][g >> 1]) : bf16_lo(sv[p][t][g >> 1]); };
+  auto offset = [&](int p, int t, int g) { return (g & 1) ? bf16_hi(bv[p][t][g >> 1]) : bf16_lo(bv[p][t][g >> 1]); };
+  if constexpr (DEQ) {
+#pragma unroll
+    for (int j = 0; j < SU; ++j) {
+      bf16x8 A[MTW][2];
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) A[mt][h] = __builtin_bit_cast(bf16x8, load_a(mt, j, h));
+#pragma unroll
+      for (int p = 0; p < NMAT; ++p)
+#pragma unroll
+        for (int t = 0; t < NTT; ++t) {
+          bf16x8 B[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int g = (2 * j + h) / GM;
+            const float s = scale(p, t, g), b = offset(p, t, g);
+            if constexpr (BITS == 8) B[h] = deq_frag8(wv[j][p][t].v[2 * h], wv[j][p][t].v[2 * h + 1], s, b);
+            else B[h] = deq_frag4(wv[j][p][t].v[h], s, s * 0.0625f, b);
+          }
+#pragma unroll
+          for (int mt = 0; mt < MTW; ++mt) {
+            acc[p][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt][0], B[0], acc[p][mt][t], 0, 0, 0);
+            acc[p][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt][1], B[1], acc[p][mt][t], 0, 0, 0);
+          }
+        }
+    }
+  } else {
+    const bf16x8 ones = as_bf16x8(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
+    float xsel[MTW] = {}, bsel[NMAT][NTT] = {};
+    // Sums and products of a group and of the one before it, whose corrections run
+    // under this one's MFMAs (the MoE gate/up walk then waits out 110 MFMA hazards a
+    // step pair instead of 160: 100 tokens over 512 experts 126 -> 122 us).
+    f32x4 xr[2][MTW], P[2][NMAT][MTW][NTT];
+    auto correct = [&](int g) {
+      const int o = g & 1;
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt)
+        if constexpr (FOLD) xsel[mt] = qmvs_pick(g, xr[o][mt][0], xsel[mt]);
+#pragma unroll
+      for (int p = 0; p < NMAT; ++p)
+#pragma unroll
+        for (int t = 0; t < NTT; ++t) {
+          const float s = scale(p, t, g), b = offset(p, t, g);
+          const float bo = OFF == 0.f ? b : __builtin_fmaf(-OFF, s, b);
+          if constexpr (FOLD) bsel[p][t] = qmvs_pick(g, bo, bsel[p][t]);
+#pragma unroll
+          for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              acc[p][mt][t][r] = __builtin_fmaf(
+                  s, P[o][p][mt][t][r],
+                  FOLD ? acc[p][mt][t][r] : __builtin_fmaf(bo, xr[o][mt][r], acc[p][mt][t][r]));
+        }
+      // The folded bias terms: after every fourth group, and after the step's last.
+      if (FOLD && ((g & 3) == 3 || g == GPS - 1)) {
+#pragma unroll
+        for (int p = 0; p < NMAT; ++p)
+#pragma unroll
+          for (int mt = 0; mt < MTW; ++mt)
+#pragma unroll
+            for (int t = 0; t < NTT; ++t)
+              acc[p][mt][t] = qmvs_bias4(xsel[mt], bsel[p][t], acc[p][mt][t]);
+      }
+    };
+#pragma unroll
+    for (int mi = 0; mi < 2 * SU; ++mi) {
+      const int j = mi >> 1, h = mi & 1, g = mi / GM, o = g & 1;
+      const bool first = mi % GM == 0, last = mi % GM == GM - 1;
+      bf16x8 A[MTW];
+#pragma unroll
+      for (int mt = 0; mt < MTW; ++mt) {
+        const u32x4 raw = load_a(mt, j, h);
+        A[mt] = BITS == 8 ? __builtin_bit_cast(bf16x8, raw) : xfrag4(raw);
+        // Sum of the x rows over the group: rows 4 (l / 16) + r of the accumulator;
+        // with FOLD row l % 16.
+        const f32x4 c = first ? f32x4{} : xr[o][mt];
+        xr[o][mt] = FOLD ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, A[mt], c, 0, 0, 0)
+                         : __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt], ones, c, 0, 0, 0);
+      }
+#pragma unroll
+      for (int p = 0; p < NMAT; ++p)
+#pragma unroll
+        for (int t = 0; t < NTT; ++t) {
+          const bf16x8 B = qmvs_bfrag<BITS>(&wv[j][p][t].v[h * (BITS / 4)]);
+#pragma unroll
+          for (int mt = 0; mt < MTW; ++mt)
+            P[o][p][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                A[mt], B, first ? f32x4{} : P[o][p][mt][t], 0, 0, 0);
+        }
+      if (last && g > 0) correct(g - 1);
+    }
+    correct(GPS - 1);
+  }
+}
 
 // w, sc, bi: the NMAT matrices ([N, K/8] u32, [N, K/64] bf16 x2).  stage: this
 // wave's NMAT * STAGE bytes of LDS.  xrow: per-lane x row pointers (see above).
@@ -305,11 +480,14 @@ constexpr int kXStageRow = 512;
 // permutation, for 22 VALU per packed word instead of 7.  The word's VALU is
 // shared by the MTW x tiles, so it pays from 2 tiles (17 to 64 x rows).
 //
-// BITS = 8 (with DEQ only): 256-byte row slices per step (16-chunk stage rows), and
-// lane (c, q) reads chunk 4 j + q of its row's unit j, the 16 values that its two
-// MFMAs of the unit take (words 0-1 and 2-3, deq_frag8); the x fragments are those
-// of the int4 walk.
-template <int MTW, int MT, int NTT, int NMAT, int WV, bool FOLD, bool DEQ = false, int BITS = 4>
+// BITS = 8: 256-byte row slices per step (16-chunk stage rows), and lane (c, q) reads
+// chunk 4 j + q of its row's unit j, the 16 values that its two MFMAs of the unit
+// take (words 0-1 and 2-3); x in natural order.
+// GS: the group size, 32, 64 or 128.  The step stays 256 values; its GPS = 256 / GS
+// scales and biases of a row are one 16-, 8- or 4-byte load, and groups of 32 order
+// K so that each MFMA stays inside one group (qmvs_xchunk).
+template <int MTW, int MT, int NTT, int NMAT, int WV, bool FOLD, bool DEQ = false, int BITS = 4,
+          int GS = 64>
 __device__ __forceinline__ void qmvs_walk_xlds(uint8_t* xs0, uint8_t* xs1, uint8_t* stage,
                                                __amdgpu_buffer_rsrc_t xres,
                                                const uint32_t (&xo)[8 * MTW / WV], int wave,
@@ -320,17 +498,15 @@ __device__ __forceinline__ void qmvs_walk_xlds(uint8_t* xs0, uint8_t* xs1, uint8
                                                int64_t N, int64_t K, int64_t s0, int64_t s1,
                                                f32x4 (&acc)[NMAT][MT][NTT]) {
   constexpr int SU = 4;
-  using G = QmvsGeom<NTT, SU, BITS>;
-  constexpr int NI = G::NI, LPR = G::LPR, RB = G::RB, ROWS = G::ROWS, SPL = G::SPL;
+  using G = QmvsGeom<NTT, SU, BITS, GS>;
+  constexpr int NI = G::NI, LPR = G::LPR, RB = G::RB, ROWS = G::ROWS, GPS = G::GPS;
   constexpr int AX = 8 * MTW / WV;
   static_assert(MTW <= MT, "walked tiles");
   static_assert(AX >= 1 && AX * WV == 8 * MTW, "x DMA split over the block's waves");
-  static_assert(BITS == 4 || (BITS == 8 && DEQ), "int8 weights are dequantized");
-  using wv_t = std::conditional_t<BITS == 8, u32x4, u32x2>;
-  typedef uint32_t sbv_t __attribute__((ext_vector_type(SPL / 2)));
+  typedef uint32_t sbv_t __attribute__((ext_vector_type(GPS / 2)));
   const int lane = threadIdx.x & 63;
   const int c16 = lane & 15, q = lane >> 4;
-  const int64_t wpr = K * BITS / 32, gpr = K / 64;
+  const int64_t wpr = K * BITS / 32, gpr = K / GS;
 
   // Weights through buffer resources as in qmvs_slice: steps past s1 load zeros
   // without a memory access.
@@ -348,28 +524,27 @@ __device__ __forceinline__ void qmvs_walk_xlds(uint8_t* xs0, uint8_t* xs1, uint8
 #pragma unroll
   for (int p = 0; p < NMAT; ++p)
     wres[p] = __builtin_amdgcn_make_buffer_rsrc((void*)w[p], (short)0, (int)(N * wpr * 4), 0x00020000);
-  int wr[NTT][SU];
+  int wr[NTT][SU][2];
 #pragma unroll
   for (int t = 0; t < NTT; ++t)
 #pragma unroll
-    for (int j = 0; j < SU; ++j) {
-      const int r = 16 * t + c16;
-      wr[t][j] = BITS == 8 ? r * RB + (qmvs_pos<RB / 32>(4 * j + q, r) << 4)
-                           : r * RB + (qmvs_pos<RB / 32>(2 * j + (q >> 1), r) << 4) + (q & 1) * 8;
-    }
-  // Scale/bias loads.  16-row tiles (NTT = 1): one 8-byte load per lane covers two
-  // steps (lane -> row l % 16, kind (l / 16) & 1 (scales, biases), step l / 32 of
-  // the pair: that step's 4 groups), issued in even steps (counted from s0) for
-  // the next pair; a lane's step is clamped to s1 - 1, so an odd step count reads
-  // no further.
-  // 32-row tiles: one load per lane and step as in qmvs_slice.
+    for (int j = 0; j < SU; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int r = 16 * t + c16;
+        wr[t][j][h] = r * RB + qmvs_woff<BITS, GS, RB>(j, h, q, r);
+      }
+  // Scale/bias loads.  16-row tiles (NTT = 1): one load per lane (8 bytes for groups
+  // of 64) covers two steps (lane -> row l % 16, kind (l / 16) & 1 (scales, biases),
+  // step l / 32 of the pair: that step's GPS groups), issued in even steps (counted
+  // from s0) for the next pair; a lane's step is clamped to s1 - 1, so an odd step
+  // count reads no further.
+  // 32-row tiles: one load per lane and step (lane -> row l % 32, kind l / 32).
   constexpr bool PAIR = ROWS == 16;
-  typedef uint32_t spv_t __attribute__((ext_vector_type(2)));
   const int sh = lane / ROWS;
   int64_t nrow = nb + lane % ROWS;
   nrow = nrow < N ? nrow : N - 1;
-  const int64_t soff =
-      nrow * gpr + ((PAIR || 64 / ROWS == 2) ? 0 : (sh >> 1) * SPL);
+  const int64_t soff = nrow * gpr;
   const uint16_t* sbrow[NMAT];
 #pragma unroll
   for (int p = 0; p < NMAT; ++p) sbrow[p] = ((sh & 1) ? bi[p] : sc[p]) + soff;
@@ -379,11 +554,11 @@ __device__ __forceinline__ void qmvs_walk_xlds(uint8_t* xs0, uint8_t* xs1, uint8
 #pragma unroll
   for (int j = 0; j < SU; ++j)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) xa[j][h] = c16 * kXStageRow + (((8 * j + 2 * q + h) ^ c16) << 4);
+    for (int h = 0; h < 2; ++h) xa[j][h] = c16 * kXStageRow + ((qmvs_xchunk<GS>(j, h, q) ^ c16) << 4);
 
   u32x4 wbuf[2][NMAT][NI];
   sbv_t sbuf[2][NMAT];
-  spv_t sp[NMAT], held[NMAT];
+  sbv_t sp[NMAT], held[NMAT];
   // Weights (and, without PAIR, the step's scales) of step st into set d; with PAIR
   // and pair set, the scales of steps st and st + 1 after the weights.
   auto load_w = [&](int d, int64_t st, bool pair) {
@@ -397,14 +572,14 @@ __device__ __forceinline__ void qmvs_walk_xlds(uint8_t* xs0, uint8_t* xs1, uint8
             u32x4, __builtin_amdgcn_raw_buffer_load_b128(
                        wres[p], past ? (int)0x80000000u : (int)(wq[i] + (uint32_t)st * RB), 0,
                        2 /* nt */));
-      if constexpr (!PAIR) sbuf[d][p] = *reinterpret_cast<const sbv_t*>(sbrow[p] + st * SU);
+      if constexpr (!PAIR) sbuf[d][p] = *reinterpret_cast<const sbv_t*>(sbrow[p] + st * GPS);
     }
     if constexpr (PAIR) {
       if (pair) {
         int64_t sl = st + ph;
         sl = sl < s1 ? sl : s1 - 1;
 #pragma unroll
-        for (int p = 0; p < NMAT; ++p) sp[p] = *reinterpret_cast<const spv_t*>(sbrow[p] + sl * SU);
+        for (int p = 0; p < NMAT; ++p) sp[p] = *reinterpret_cast<const sbv_t*>(sbrow[p] + sl * GPS);
       }
     }
   };
@@ -445,15 +620,15 @@ __device__ __forceinline__ void qmvs_walk_xlds(uint8_t* xs0, uint8_t* xs1, uint8
 #pragma unroll
       for (int i = 0; i < NI; ++i)
         *reinterpret_cast<u32x4*>(stage + p * G::STAGE + wo[i]) = wbuf[e][p][i];
-    wv_t wv[SU][NMAT][NTT];
+    QmvsWords<BITS, GS> wv[SU][NMAT][NTT];
 #pragma unroll
     for (int j = 0; j < SU; ++j)
 #pragma unroll
       for (int p = 0; p < NMAT; ++p)
 #pragma unroll
         for (int t = 0; t < NTT; ++t)
-          wv[j][p][t] = *reinterpret_cast<const wv_t*>(stage + p * G::STAGE + wr[t][j]);
-    uint32_t sv[NMAT][NTT][SU / 2], bv[NMAT][NTT][SU / 2];
+          wv[j][p][t] = qmvs_read_words<BITS, GS>(stage + p * G::STAGE, wr[t][j][0], wr[t][j][1]);
+    uint32_t sv[NMAT][NTT][GPS / 2], bv[NMAT][NTT][GPS / 2];
     if constexpr (PAIR) {
       if constexpr (e == 0) {
 #pragma unroll
@@ -462,7 +637,7 @@ __device__ __forceinline__ void qmvs_walk_xlds(uint8_t* xs0, uint8_t* xs1, uint8
 #pragma unroll
       for (int p = 0; p < NMAT; ++p)
 #pragma unroll
-        for (int k = 0; k < SU / 2; ++k) {
+        for (int k = 0; k < GPS / 2; ++k) {
           sv[p][0][k] = (uint32_t)__shfl((int)held[p][k], 32 * e + c16, 64);
           bv[p][0][k] = (uint32_t)__shfl((int)held[p][k], 32 * e + 16 + c16, 64);
         }
@@ -475,12 +650,10 @@ __device__ __forceinline__ void qmvs_walk_xlds(uint8_t* xs0, uint8_t* xs1, uint8
 #pragma unroll
         for (int t = 0; t < NTT; ++t)
 #pragma unroll
-          for (int k = 0; k < SU / 2; ++k) {
+          for (int k = 0; k < GPS / 2; ++k) {
             const int row = 16 * t + c16;
-            const int hi = (64 / ROWS == 2) ? 0 : k / (SPL / 2);
-            const int idx = (64 / ROWS == 2) ? k : k % (SPL / 2);
-            sv[p][t][k] = (uint32_t)__shfl((int)mine[p][idx], (2 * hi) * ROWS + row, 64);
-            bv[p][t][k] = (uint32_t)__shfl((int)mine[p][idx], (2 * hi + 1) * ROWS + row, 64);
+            sv[p][t][k] = (uint32_t)__shfl((int)mine[p][k], row, 64);
+            bv[p][t][k] = (uint32_t)__shfl((int)mine[p][k], ROWS + row, 64);
           }
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -488,89 +661,11 @@ __device__ __forceinline__ void qmvs_walk_xlds(uint8_t* xs0, uint8_t* xs1, uint8
     __builtin_amdgcn_sched_barrier(0);
     load_w(e, stp + 2, e == 0);
     __builtin_amdgcn_sched_barrier(0);
-    float xsel[MTW] = {}, bsel[NMAT][NTT] = {};
-    f32x4 xr[MTW];
-#pragma unroll
-    for (int j = 0; j < SU; ++j) {
-      if constexpr (DEQ) {
-        static_assert(!FOLD, "DEQ accumulates the dequantized product directly");
-        bf16x8 A[MTW][2];
-#pragma unroll
-        for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            A[mt][h] = __builtin_bit_cast(
-                bf16x8, *reinterpret_cast<const u32x4*>(xc + mt * 16 * kXStageRow + xa[j][h]));
-#pragma unroll
-        for (int p = 0; p < NMAT; ++p)
-#pragma unroll
-          for (int t = 0; t < NTT; ++t) {
-            const float s = (j & 1) ? bf16_hi(sv[p][t][j >> 1]) : bf16_lo(sv[p][t][j >> 1]);
-            const float b = (j & 1) ? bf16_hi(bv[p][t][j >> 1]) : bf16_lo(bv[p][t][j >> 1]);
-            bf16x8 B0, B1;
-            if constexpr (BITS == 8) {
-              B0 = deq_frag8(wv[j][p][t][0], wv[j][p][t][1], s, b);
-              B1 = deq_frag8(wv[j][p][t][2], wv[j][p][t][3], s, b);
-            } else {
-              B0 = deq_frag4(wv[j][p][t][0], s, s * 0.0625f, b);
-              B1 = deq_frag4(wv[j][p][t][1], s, s * 0.0625f, b);
-            }
-#pragma unroll
-            for (int mt = 0; mt < MTW; ++mt) {
-              acc[p][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt][0], B0, acc[p][mt][t], 0, 0, 0);
-              acc[p][mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt][1], B1, acc[p][mt][t], 0, 0, 0);
-            }
-          }
-        continue;
-      }
-      bf16x8 A[MTW][2];
-#pragma unroll
-      for (int mt = 0; mt < MTW; ++mt) {
-        A[mt][0] = xfrag4(*reinterpret_cast<const u32x4*>(xc + mt * 16 * kXStageRow + xa[j][0]));
-        A[mt][1] = xfrag4(*reinterpret_cast<const u32x4*>(xc + mt * 16 * kXStageRow + xa[j][1]));
-      }
-#pragma unroll
-      for (int mt = 0; mt < MTW; ++mt) {
-        if constexpr (FOLD) xsel[mt] = qmvs_pick(j, qmvs_xsum(A[mt]), xsel[mt]);
-        else xr[mt] = qmvs_xsum_rows(A[mt]);
-      }
-#pragma unroll
-      for (int p = 0; p < NMAT; ++p) {
-        f32x4 P[MTW][NTT];
-#pragma unroll
-        for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-          for (int t = 0; t < NTT; ++t) {
-            P[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                A[mt][0], wfrag<4>(wv[j][p][t][0]), f32x4{}, 0, 0, 0);
-            P[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                A[mt][1], wfrag<4>(wv[j][p][t][1]), P[mt][t], 0, 0, 0);
-          }
-#pragma unroll
-        for (int t = 0; t < NTT; ++t) {
-          const float s = (j & 1) ? bf16_hi(sv[p][t][j >> 1]) : bf16_lo(sv[p][t][j >> 1]);
-          const float b = (j & 1) ? bf16_hi(bv[p][t][j >> 1]) : bf16_lo(bv[p][t][j >> 1]);
-          const float bo = __builtin_fmaf(-128.f, s, b);
-          if constexpr (FOLD) bsel[p][t] = qmvs_pick(j, bo, bsel[p][t]);
-#pragma unroll
-          for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              acc[p][mt][t][r] = __builtin_fmaf(
-                  s, P[mt][t][r],
-                  FOLD ? acc[p][mt][t][r] : __builtin_fmaf(bo, xr[mt][r], acc[p][mt][t][r]));
-        }
-      }
-      if (FOLD && (j & 3) == 3) {
-#pragma unroll
-        for (int p = 0; p < NMAT; ++p)
-#pragma unroll
-          for (int mt = 0; mt < MTW; ++mt)
-#pragma unroll
-            for (int t = 0; t < NTT; ++t)
-              acc[p][mt][t] = qmvs_bias4(xsel[mt], bsel[p][t], acc[p][mt][t]);
-      }
-    }
+    qmvs_step_mma<MTW, MT, NTT, NMAT, SU, FOLD, DEQ, BITS, GS>(
+        [&](int mt, int j, int h) {
+          return *reinterpret_cast<const u32x4*>(xc + mt * 16 * kXStageRow + xa[j][h]);
+        },
+        wv, sv, bv, acc);
   };
   int64_t st = s0;
 #pragma clang loop unroll(disable)
@@ -595,25 +690,24 @@ __device__ __forceinline__ void qmvs_walk_xlds(uint8_t* xs0, uint8_t* xs1, uint8
 // a memory access) and are not computed.
 // DEQ: the weights dequantized and x in natural order, as in qmvs_walk_xlds, and
 // BITS = 8 with it as there.
-template <int MT, int NTT, int WV, int D, bool DEQ = false, int BITS = 4>
+template <int MT, int NTT, int WV, int D, bool DEQ = false, int BITS = 4, int GS = 64>
 __device__ __forceinline__ void qmvs_walk_xall(uint8_t* xs, uint8_t* stage, __amdgpu_buffer_rsrc_t xres,
                                                const uint32_t (&xo)[8 * MT / WV], int wave,
                                                const uint32_t* w, const uint16_t* sc,
                                                const uint16_t* bi, int64_t nb, int64_t N, int64_t K,
-                                               int64_t s0, int64_t s1, f32x4 (&acc)[MT][NTT]) {
+                                               int64_t s0, int64_t s1, f32x4 (&acc)[1][MT][NTT]) {
   constexpr int SU = 4;
-  using G = QmvsGeom<NTT, SU, BITS>;
+  using G = QmvsGeom<NTT, SU, BITS, GS>;
   constexpr int NI = G::NI, LPR = G::LPR, RB = G::RB, ROWS = G::ROWS, SPL = G::SPL;
+  constexpr int GPS = G::GPS;
   constexpr int AX = 8 * MT / WV;
   constexpr int XSLOT = 16 * MT * kXStageRow;
   static_assert(AX >= 1 && AX * WV == 8 * MT, "x DMA split over the block's waves");
   static_assert(D >= 1 && D * NI < 64, "vmcnt range");
-  static_assert(BITS == 4 || (BITS == 8 && DEQ), "int8 weights are dequantized");
-  using wv_t = std::conditional_t<BITS == 8, u32x4, u32x2>;
   typedef uint32_t sbv_t __attribute__((ext_vector_type(SPL / 2)));
   const int lane = threadIdx.x & 63;
   const int c16 = lane & 15, q = lane >> 4;
-  const int64_t wpr = K * BITS / 32, gpr = K / 64;
+  const int64_t wpr = K * BITS / 32, gpr = K / GS;
   if (s1 <= s0) return;
 
   uint32_t wq[NI];
@@ -628,26 +722,27 @@ __device__ __forceinline__ void qmvs_walk_xall(uint8_t* xs, uint8_t* stage, __am
   }
   const __amdgpu_buffer_rsrc_t wres =
       __builtin_amdgcn_make_buffer_rsrc((void*)w, (short)0, (int)(N * wpr * 4), 0x00020000);
-  int wr[NTT][SU];
+  int wr[NTT][SU][2];
 #pragma unroll
   for (int t = 0; t < NTT; ++t)
 #pragma unroll
-    for (int j = 0; j < SU; ++j) {
-      const int r = 16 * t + c16;
-      wr[t][j] = BITS == 8 ? r * RB + (qmvs_pos<RB / 32>(4 * j + q, r) << 4)
-                           : r * RB + (qmvs_pos<RB / 32>(2 * j + (q >> 1), r) << 4) + (q & 1) * 8;
-    }
+    for (int j = 0; j < SU; ++j)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int r = 16 * t + c16;
+        wr[t][j][h] = r * RB + qmvs_woff<BITS, GS, RB>(j, h, q, r);
+      }
   // Scale/bias words as in qmvs_slice: lane -> row l % ROWS, kind (l / ROWS) & 1,
   // and for 16-row tiles which half of the step's groups (l / ROWS / 2).
   const int sh = lane / ROWS;
   int64_t nrow = nb + lane % ROWS;
   nrow = nrow < N ? nrow : N - 1;
-  const uint16_t* sbrow = ((sh & 1) ? bi : sc) + nrow * gpr + ((64 / ROWS == 2) ? 0 : (sh >> 1) * SPL);
+  const uint16_t* sbrow = ((sh & 1) ? bi : sc) + nrow * gpr + (G::HALVES == 2 ? (sh >> 1) * SPL : 0);
   int xa[SU][2];
 #pragma unroll
   for (int j = 0; j < SU; ++j)
 #pragma unroll
-    for (int h = 0; h < 2; ++h) xa[j][h] = c16 * kXStageRow + (((8 * j + 2 * q + h) ^ c16) << 4);
+    for (int h = 0; h < 2; ++h) xa[j][h] = c16 * kXStageRow + ((qmvs_xchunk<GS>(j, h, q) ^ c16) << 4);
 
   // Issue order: scale/bias words, x DMAs, weights.  The wait for x then counts
   // only the weight loads (16-byte loads, which the compiler cannot merge), however
@@ -657,7 +752,7 @@ __device__ __forceinline__ void qmvs_walk_xall(uint8_t* xs, uint8_t* stage, __am
 #pragma unroll
   for (int d = 0; d < D; ++d) {
     const int64_t st = s0 + d < s1 ? s0 + d : s1 - 1;
-    sbuf[d] = *reinterpret_cast<const sbv_t*>(sbrow + st * SU);
+    sbuf[d] = *reinterpret_cast<const sbv_t*>(sbrow + st * GPS);
   }
   __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -685,7 +780,6 @@ __device__ __forceinline__ void qmvs_walk_xall(uint8_t* xs, uint8_t* stage, __am
   qmvs_wait_vm_lgkm0<D * NI>();
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_sched_barrier(0);
-  const bf16x8 ones = as_bf16x8(0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u);
 
 #pragma unroll
   for (int d = 0; d < D; ++d) {
@@ -694,87 +788,27 @@ __device__ __forceinline__ void qmvs_walk_xall(uint8_t* xs, uint8_t* stage, __am
 #pragma unroll
     for (int i = 0; i < NI; ++i)
       *reinterpret_cast<u32x4*>(stage + wo[i]) = wbuf[d][i];
-    wv_t wv[SU][NTT];
+    QmvsWords<BITS, GS> wv[SU][1][NTT];
 #pragma unroll
     for (int j = 0; j < SU; ++j)
 #pragma unroll
       for (int t = 0; t < NTT; ++t)
-        wv[j][t] = *reinterpret_cast<const wv_t*>(stage + wr[t][j]);
-    uint32_t sv[NTT][SU / 2], bv[NTT][SU / 2];
+        wv[j][0][t] = qmvs_read_words<BITS, GS>(stage, wr[t][j][0], wr[t][j][1]);
+    uint32_t sv[1][NTT][GPS / 2], bv[1][NTT][GPS / 2];
 #pragma unroll
     for (int t = 0; t < NTT; ++t)
 #pragma unroll
-      for (int k = 0; k < SU / 2; ++k) {
+      for (int k = 0; k < GPS / 2; ++k) {
         const int row = 16 * t + c16;
-        const int hi = (64 / ROWS == 2) ? 0 : k / (SPL / 2);
-        const int idx = (64 / ROWS == 2) ? k : k % (SPL / 2);
-        sv[t][k] = (uint32_t)__shfl((int)sbuf[d][idx], (2 * hi) * ROWS + row, 64);
-        bv[t][k] = (uint32_t)__shfl((int)sbuf[d][idx], (2 * hi + 1) * ROWS + row, 64);
+        const int hi = k / (SPL / 2), idx = k % (SPL / 2);
+        sv[0][t][k] = (uint32_t)__shfl((int)sbuf[d][idx], (2 * hi) * ROWS + row, 64);
+        bv[0][t][k] = (uint32_t)__shfl((int)sbuf[d][idx], (2 * hi + 1) * ROWS + row, 64);
       }
-#pragma unroll
-    for (int j = 0; j < SU; ++j) {
-      if constexpr (DEQ) {
-        bf16x8 A[MT][2];
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-          for (int h = 0; h < 2; ++h)
-            A[mt][h] = __builtin_bit_cast(
-                bf16x8, *reinterpret_cast<const u32x4*>(xc + mt * 16 * kXStageRow + xa[j][h]));
-#pragma unroll
-        for (int t = 0; t < NTT; ++t) {
-          const float sf = (j & 1) ? bf16_hi(sv[t][j >> 1]) : bf16_lo(sv[t][j >> 1]);
-          const float bf = (j & 1) ? bf16_hi(bv[t][j >> 1]) : bf16_lo(bv[t][j >> 1]);
-          bf16x8 B0, B1;
-          if constexpr (BITS == 8) {
-            B0 = deq_frag8(wv[j][t][0], wv[j][t][1], sf, bf);
-            B1 = deq_frag8(wv[j][t][2], wv[j][t][3], sf, bf);
-          } else {
-            B0 = deq_frag4(wv[j][t][0], sf, sf * 0.0625f, bf);
-            B1 = deq_frag4(wv[j][t][1], sf, sf * 0.0625f, bf);
-          }
-#pragma unroll
-          for (int mt = 0; mt < MT; ++mt) {
-            acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt][0], B0, acc[mt][t], 0, 0, 0);
-            acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt][1], B1, acc[mt][t], 0, 0, 0);
-          }
-        }
-        continue;
-      }
-      bf16x8 A[MT][2];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        A[mt][0] = xfrag4(*reinterpret_cast<const u32x4*>(xc + mt * 16 * kXStageRow + xa[j][0]));
-        A[mt][1] = xfrag4(*reinterpret_cast<const u32x4*>(xc + mt * 16 * kXStageRow + xa[j][1]));
-      }
-      f32x4 xsum[MT];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        xsum[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt][0], ones, f32x4{}, 0, 0, 0);
-        xsum[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt][1], ones, xsum[mt], 0, 0, 0);
-      }
-      f32x4 P[MT][NTT];
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int t = 0; t < NTT; ++t) {
-          P[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt][0], wfrag<4>(wv[j][t][0]),
-                                                             f32x4{}, 0, 0, 0);
-          P[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[mt][1], wfrag<4>(wv[j][t][1]),
-                                                             P[mt][t], 0, 0, 0);
-        }
-#pragma unroll
-      for (int t = 0; t < NTT; ++t) {
-        const float sf = (j & 1) ? bf16_hi(sv[t][j >> 1]) : bf16_lo(sv[t][j >> 1]);
-        const float bf = (j & 1) ? bf16_hi(bv[t][j >> 1]) : bf16_lo(bv[t][j >> 1]);
-        const float bo = __builtin_fmaf(-128.f, sf, bf);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            acc[mt][t][r] = __builtin_fmaf(sf, P[mt][t][r], __builtin_fmaf(bo, xsum[mt][r], acc[mt][t][r]));
-      }
-    }
+    qmvs_step_mma<MT, MT, NTT, 1, SU, false, DEQ, BITS, GS>(
+        [&](int mt, int j, int h) {
+          return *reinterpret_cast<const u32x4*>(xc + mt * 16 * kXStageRow + xa[j][h]);
+        },
+        wv, sv, bv, acc);
   }
 }
 

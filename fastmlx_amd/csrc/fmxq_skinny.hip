@@ -423,7 +423,7 @@ void qmvw_kernel(QmmArgs a) {
   if constexpr (D > 0) {
     qmvs_walk_xall<MT, NTT, WV, D, kDeqXall, BITS>(&xs[0][0], stage[wave], xres, xo, wave,
                                                               a.w, a.scales, a.biases,
-                                   nb, a.N, a.K, s0, s1, acc[0]);
+                                   nb, a.N, a.K, s0, s1, acc);
   } else {
     const uint32_t* const w[1] = {a.w};
     const uint16_t* const sc[1] = {a.scales};

@@ -844,6 +844,82 @@ def test_moe_layer_gated_shared_expert(gpu, oracle, T, E, D, k):
                          what=f"moe_layer gated T={T}")
 
 
+# --- the weight formats other than 4 bits in groups of 64 ---
+
+@pytest.mark.parametrize("bits,group", [(4, 32), (4, 128), (8, 32), (8, 64), (8, 128)])
+@pytest.mark.parametrize("E,T,k,D,I,bad", [
+    (5, 1, 3, 2048, 768, False),   # one token: GEMV, down rows that leave lanes idle
+    (5, 5, 3, 512, 512, True),     # 15 slots below the GEMV's depth: the walk without a sort
+    (64, 6, 5, 2304, 256, True),   # few slots per expert: GEMV, fused combine, one short slice
+    (16, 10, 3, 768, 256, False),  # sorted, 16-slot pieces, three steps; one-step down walk
+    (3, 40, 2, 1024, 1280, True),  # sorted, 32-slot pieces longer than 16; five steps
+    (4, 3, 3, 8448, 512, False),   # GEMV rows in 8 and 16 slices
+])
+def test_moe_layer_formats(gpu, oracle, bits, group, E, T, k, D, I, bad):
+    """The layer with a gated shared expert in each weight format, through every route of
+    the walk and the GEMV, against the exact-affine oracle (the bounds of
+    tests/parity.py: these formats dequantize nothing to bf16)."""
+    from fastmlx_amd import FmxqError, ops
+
+    rng = np.random.default_rng(bits * 1000 + group + D + I)
+    gate, up, down = _stack(rng, E, D, I, bits, group)
+    sh = _stack(rng, 1, D, I, bits, group)
+    x = make_x(rng, T, D)
+    inds = topk_uniform(rng, T, E, k)
+    if bad:
+        inds[T // 2, 1] = E + 3
+    w16 = oracle.f32_to_bf16(rng.dirichlet(np.ones(k), size=T).astype(np.float32))
+    sg = make_x(rng, T)
+    dev = lambda t: to_dev(t, gpu)
+    dstack = [tuple(map(dev, m)) for m in (gate, up, down)]
+    di = dev(inds.astype(np.uint32))
+    announce(f"moe_layer {bits}-bit group {group} E={E} T={T} k={k} D={D} I={I}")
+    ys = ops.switch_glu(dev(x), di, *dstack, group, bits)
+    out = ops.moe_layer(dev(x), di, *dstack, dev(w16), [tuple(map(dev, m)) for m in sh], dev(sg),
+                        group, bits)
+    torch.cuda.synchronize()
+    if bad:
+        with pytest.raises(FmxqError):
+            ops.device_error()
+    else:
+        ops.device_error()
+    ok = inds < E
+    sref = parity.SwitchRef(x, np.where(ok, inds, 0), gate, up, down, group, bits, fused=False)
+    got = to_np(ys)
+    assert np.all(got[~ok] == 0)
+    parity.check_switch(got[ok], sref.masked(ok), what="switch_glu")
+    near = sref.refs[0] * ok[:, :, None]
+    allow = parity.switch_bound(near, near, sref.hscale) * ok[:, :, None]
+    ssref = parity.SwitchRef(x, np.zeros((T, 1), np.int32), *sh, group, bits, fused=False)
+    sv = ssref.refs[0][:, 0]
+    sa = parity.switch_bound(ssref.refs[0], ssref.refs[0], ssref.hscale)[:, 0]
+    gt = 1 / (1 + np.exp(-oracle.bf16_to_f32(sg).astype(np.float64)))[:, None]
+    # The gate and the gated row are each rounded to bf16 once: 2^-8 of the row apiece.
+    parity.combine_check(to_np(out), near, allow, w16,
+                         shared=(gt * sv, gt * sa + 2.0 ** -7 * np.abs(gt * sv)), what="moe_layer")
+
+
+@pytest.mark.parametrize("bits,group", [(4, 32), (8, 64), (8, 128)])
+def test_gather_qmm_formats(gpu, oracle, bits, group):
+    """gather_qmm's sorted items in runs of 1, 16, 17, 33 and 40, the last expert unused."""
+    from fastmlx_amd import ops
+
+    rng = np.random.default_rng(bits + group)
+    E, N, K = 7, 200, 1280
+    w, s, b = make_quant(rng, (E, N), K, bits, group)
+    rhs = np.repeat([0, 1, 2, 4, 5], [1, 16, 17, 33, 40]).astype(np.uint32)
+    lhs = rng.permutation(len(rhs)).astype(np.uint32)
+    x = make_x(rng, len(rhs), 1, K)
+    dev = lambda t: to_dev(t, gpu)
+    announce(f"gather_qmm {bits}-bit group {group}")
+    y = ops.gather_qmm(dev(x), dev(w), dev(s), dev(b), dev(rhs), dev(lhs), 1, True, group, bits, True)
+    torch.cuda.synchronize()
+    ops.device_error()
+    ref = parity.gather_refs(x.reshape(-1, K), w, s, b, lhs.astype(np.int32),
+                             rhs.astype(np.int32), group, bits)
+    parity.check_dense(to_np(y).reshape(-1, N), ref, what="gather_qmm")
+
+
 @pytest.mark.parametrize("T", [1, 20])
 def test_moe_layer_bad_expert_id(gpu, oracle, T):
     """Bad routed ids: their slots contribute zero, the shared expert and the other
