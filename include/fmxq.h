@@ -157,8 +157,8 @@ int fmxq_switch_glu(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
  * (qwen3next_forward.go:510-525, deepseekv3_forward.go:427-442).  Arguments are
  * those of the two calls; the op chain and its bf16 roundings are theirs.  Up to
  * 16 routing slots, and up to 256 slots routed over at least twice as many
- * experts (int4, group 64), the slots stay unsorted and the down projection and
- * the weighted sum run as one kernel; otherwise the expert rows go through a
+ * experts, the slots stay unsorted and the down projection and the weighted sum
+ * run as one kernel (any supported format, I a multiple of 256); otherwise the expert rows go through a
  * per-stream buffer. */
 int fmxq_switch_glu_combine(const uint16_t* x, const uint32_t* inds, const uint32_t* w_gate,
                             const uint16_t* s_gate, const uint16_t* b_gate,
@@ -177,8 +177,9 @@ int fmxq_switch_glu_combine(const uint16_t* x, const uint32_t* inds, const uint3
  * the shared expert's gate, up and down triples laid out as one-expert stacks
  * ([1, I, D*bits/32], [1, D, I*bits/32], ...), with the routed experts' I.  The
  * shared expert's op chain and roundings are those of a one-expert SwitchGLU.
- * For one token (decode) the shared expert runs inside the routed kernels (one
- * more gate/up segment, one more wave per down/combine block; top_k <= 15).
+ * Batches whose slots stay unsorted (see fmxq_switch_glu_combine; D in 2048..16384,
+ * top_k <= 15) run the shared expert inside the routed kernels (one more gate/up
+ * segment per token, one more wave per down/combine block).
  * Batches whose routed slots are sorted (below 4096 slots) sort it in as one
  * more expert with one slot per token, so it runs inside the routed gate/up and
  * down launches.  Otherwise it runs as fmxq_switch_glu on every token, then
