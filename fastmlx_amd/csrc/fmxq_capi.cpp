@@ -216,17 +216,19 @@ struct MoeScratch {
   uint16_t* h;
   uint32_t *tiles = nullptr, *ntile = nullptr;
   uint16_t *g = nullptr, *u = nullptr;
+  uint8_t* xprep = nullptr;  // with prep > 0: that many bytes for the tiles' x
 };
 int moe_scratch(hipStream_t s, int64_t S, int64_t h_cols, int64_t max_seg, MoeScratch* m,
                 const char* op, int64_t max_tiles = 0, int64_t gu_cols = 0,
-                const ScratchSource& src = ScratchSource()) {
+                const ScratchSource& src = ScratchSource(), int64_t prep = 0) {
   const size_t ib = align_up((size_t)S * sizeof(uint32_t));
   const size_t sb = align_up((size_t)max_seg * 2 * sizeof(uint32_t));
   const size_t hb = align_up((size_t)S * h_cols * sizeof(uint16_t));
   const size_t tb = align_up((size_t)max_tiles * 2 * sizeof(uint32_t));
   const size_t gb = align_up((size_t)S * gu_cols * sizeof(uint16_t));
   void* arena = nullptr;
-  if (int rc = src.get(s, 3 * ib + sb + 256 + hb + tb + 256 + 2 * gb, &arena, op)) return rc;
+  const size_t pb = align_up((size_t)prep);
+  if (int rc = src.get(s, 3 * ib + sb + 256 + hb + tb + 256 + 2 * gb + pb, &arena, op)) return rc;
   char* p = static_cast<char*>(arena);
   m->order = reinterpret_cast<uint32_t*>(p);
   m->rhs = reinterpret_cast<uint32_t*>(p + ib);
@@ -243,6 +245,7 @@ int moe_scratch(hipStream_t s, int64_t S, int64_t h_cols, int64_t max_seg, MoeSc
       m->u = reinterpret_cast<uint16_t*>(q + tb + 256 + gb);
     }
   }
+  m->xprep = prep > 0 ? reinterpret_cast<uint8_t*>(q + tb + 256 + 2 * gb) : nullptr;
   return FMXQ_OK;
 }
 
@@ -520,14 +523,19 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
                       group_size, bits, lhs_div};
       return hip_status(fmxq::launch_moe_qmvs(a, 1, 16, batch, s), op);
     }
-    const int window = fmxq::moe_window(batch, E);
+    const int window = fmxq::moe_window(batch, E, N, K, N, K, x_batch, bits, group_size);
     const int64_t max_seg = fmxq::moe_max_segments(batch, E, window);
     if (max_seg <= kMaxSegmentsGrid) {
       MoeScratch m;
-      const int64_t max_tiles = fmxq::qmm_grouped_supported(N, K, x_batch, bits, group_size)
+      const int64_t max_tiles = window != fmxq::kMoeTileRows &&
+                                        fmxq::qmm_grouped_supported(N, K, x_batch, bits, group_size)
                                     ? grouped_max_tiles(batch, E)
                                     : 0;
-      if (int rc = moe_scratch(s, batch, 0, max_seg, &m, op, max_tiles)) return rc;
+      const int64_t prep = window == fmxq::kMoeTileRows
+                               ? fmxq::moe_tile_prep_bytes(x_batch * K, bits, group_size)
+                               : 0;
+      if (int rc = moe_scratch(s, batch, 0, max_seg, &m, op, max_tiles, 0, ScratchSource(), prep))
+        return rc;
       if (int rc = hip_status(fmxq::launch_sort_slots(rhs_indices, batch, lhs_div, E, m.order,
                                                       m.rhs, m.lhs, s, lhs_indices, m.seg,
                                                       m.nseg, window, m.tiles, m.ntile,
@@ -537,6 +545,7 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
         return rc;
       fmxq::MoeArgs a{x, m.lhs, {w, nullptr}, {scales, nullptr}, {biases, nullptr}, m.rhs,
                       m.seg, m.nseg, y, m.order, batch, N, K, E, x_batch, flag, group_size, bits};
+      a.xprep = m.xprep;
       if (int rc = hip_status(fmxq::launch_moe_qmvs(a, 1, window, max_seg, s), op)) return rc;
       if (!max_tiles) return FMXQ_OK;
       const fmxq::QmmArgs gq = grouped_args(x, w, scales, biases, y, N, K, bits, group_size, m,
@@ -617,7 +626,18 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
   hipStream_t s = static_cast<hipStream_t>(stream);
   uint32_t* flag = nullptr;
   if (int rc = device_flag(static_cast<hipStream_t>(stream), &flag)) return rc;
-  const int window = fmxq::moe_window(S, E);
+  // The tiles keep a prepared copy of x, then of h; where the fixed scratch of the
+  // allocation-free call does not hold it, the walk takes the batch.
+  int window = fmxq::moe_window(S, E, I, D, D, I, std::max(S, T), bits, group_size);
+  int64_t prep = 0;
+  if (window == fmxq::kMoeTileRows) {
+    prep = fmxq::moe_tile_prep_bytes(std::max(T * D, S * I), bits, group_size);
+    const int64_t rest = 2 * S * I + 12 * S + 16 * (S + E) + 4096;
+    if (src.fixed && prep + rest > (int64_t)src.fixed_bytes) {
+      window = fmxq::moe_walk_window(S, E);
+      prep = 0;
+    }
+  }
   const int64_t max_seg = fmxq::moe_max_segments(S, E, window);
   if (E <= kSortMaxExperts && max_seg <= kMaxSegmentsGrid &&
       fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
@@ -642,11 +662,11 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
     // Long expert runs (>= kGroupedMinRun slots) go to the grouped GEMM: gate and
     // up into g and u, silu * up into their h rows, then down.
     const int64_t max_tiles =
-        fmxq::qmm_grouped_supported(I, D, T, bits, group_size) &&
+        window != fmxq::kMoeTileRows && fmxq::qmm_grouped_supported(I, D, T, bits, group_size) &&
                 fmxq::qmm_grouped_supported(D, I, S, bits, group_size)
             ? grouped_max_tiles(S, E)
             : 0;
-    if (int rc = moe_scratch(s, S, I, max_seg, &m, op, max_tiles, max_tiles ? I : 0, src))
+    if (int rc = moe_scratch(s, S, I, max_seg, &m, op, max_tiles, max_tiles ? I : 0, src, prep))
       return rc;
     if (int rc = hip_status(fmxq::launch_sort_slots(inds, S, topk, E, m.order, m.rhs, m.lhs, s,
                                                     nullptr, m.seg, m.nseg, window, m.tiles,
@@ -656,6 +676,7 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
       return rc;
     fmxq::MoeArgs gu{x, m.lhs, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, m.rhs, m.seg,
                      m.nseg, m.h, nullptr, S, I, D, E, T, flag, group_size, bits};
+    gu.xprep = m.xprep;
     if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, window, max_seg, s),
                             "switch_glu: gate/up"))
       return rc;
@@ -676,6 +697,7 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
     }
     fmxq::MoeArgs dn{m.h, nullptr, {w_down, nullptr}, {s_down, nullptr}, {b_down, nullptr},
                      m.rhs, m.seg, m.nseg, out, m.order, S, D, I, E, S, flag, group_size, bits};
+    dn.xprep = m.xprep;
     if (int rc = hip_status(fmxq::launch_moe_qmvs(dn, 1, window, max_seg, s), "switch_glu: down"))
       return rc;
     if (!max_tiles) return FMXQ_OK;
@@ -868,9 +890,10 @@ extern "C" int fmxq_moe_layer(
   // arena's slot 1, routed then shared, and the combine reads both.
   {
     const int64_t Sa = S + T;
-    const int window = fmxq::moe_window(Sa, E + 1);
+    const int window = fmxq::moe_window(Sa, E + 1, I, D, D, I, Sa, bits, group_size);
     const int64_t max_seg = fmxq::moe_max_segments(Sa, E + 1, window);
-    if (!fmxq::moe_combine_unsorted(S, E) && grouped_max_tiles(S, E) == 0 &&
+    if (!fmxq::moe_combine_unsorted(S, E) &&
+        (window == fmxq::kMoeTileRows || grouped_max_tiles(S, E) == 0) &&
         E + 1 <= kSortMaxExperts && max_seg <= kMaxSegmentsGrid &&
         fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
         fmxq::moe_qmvs_supported(D, I, S + T, bits, group_size) && aligned16(s_gate) &&
@@ -880,7 +903,11 @@ extern "C" int fmxq_moe_layer(
       uint32_t* flag = nullptr;
       if (int rc = device_flag(s, &flag)) return rc;
       MoeScratch m;
-      if (int rc = moe_scratch(s, Sa, I, max_seg, &m, op)) return rc;
+      const int64_t prep =
+          window == fmxq::kMoeTileRows
+              ? fmxq::moe_tile_prep_bytes(std::max(T * D, Sa * I), bits, group_size)
+              : 0;
+      if (int rc = moe_scratch(s, Sa, I, max_seg, &m, op, 0, 0, ScratchSource(), prep)) return rc;
       void* rows = nullptr;
       if (int rc = stream_arena(s, align_up((size_t)Sa * D * sizeof(uint16_t)), &rows, op, 1))
         return rc;
@@ -899,6 +926,7 @@ extern "C" int fmxq_moe_layer(
       gu.sh_b[0] = sb_gate;
       gu.sh_b[1] = sb_up;
       gu.sh_seg = true;
+      gu.xprep = m.xprep;
       if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, window, max_seg, s),
                               "moe_layer: gate/up"))
         return rc;
@@ -908,6 +936,7 @@ extern "C" int fmxq_moe_layer(
       dn.sh_s[0] = ss_down;
       dn.sh_b[0] = sb_down;
       dn.sh_seg = true;
+      dn.xprep = m.xprep;
       if (int rc = hip_status(fmxq::launch_moe_qmvs(dn, 1, window, max_seg, s), "moe_layer: down"))
         return rc;
       return hip_status(fmxq::launch_moe_combine(y, weights, y + S * D, shared_gate, out, T, topk,

@@ -269,6 +269,11 @@ struct MoeArgs {
   // Segment-table form only: expert id E names the shared expert (sh_w / sh_s /
   // sh_b), ids above E are out of range (launch_sort_slots with sh_T > 0).
   bool sh_seg = false;
+  // Tiles only: scratch of moe_tile_prep_bytes for x_rows rows of K values; the
+  // launcher points xsum and xp into it.
+  uint8_t* xprep = nullptr;
+  const uint8_t* xsum = nullptr;
+  const uint16_t* xp = nullptr;
 };
 // Slot counts up to which the MoE products skip the sort: every slot is its own
 // segment (a sort saves weight reads only when slots share an expert).
@@ -284,8 +289,23 @@ constexpr int64_t kMoeUnsortedCombineMaxSlots = 256;
 inline bool moe_combine_unsorted(int64_t S, int64_t E) {
   return S <= kMoeUnsortedMaxSlots || (S <= kMoeUnsortedCombineMaxSlots && 2 * S <= E);
 }
+constexpr int kMoeTileRows = 64;
+// Bytes of the group sums of 128 values of x (fmxq_moe_tile.hpp), of n values (16-byte
+// pieces per row and 128 values), and of everything the tiles keep about n values of x.
+constexpr int tile_sum_bytes(int group_size) { return group_size == 32 ? 32 : 16; }
+inline int64_t moe_tile_sum_bytes(int64_t n, int group_size) {
+  return (n / 128 * tile_sum_bytes(group_size) + 255) & ~int64_t(255);
+}
+inline int64_t moe_tile_prep_bytes(int64_t n, int bits, int group_size) {
+  return moe_tile_sum_bytes(n, group_size) + (bits == 4 ? 2 * n : 0);
+}
 bool moe_qmvs_supported(int64_t N, int64_t K, int64_t x_rows, int bits, int group_size);
-int moe_window(int64_t S, int64_t E);
+// Slots per segment of a sorted batch of S slots over E experts, for products of N1 x
+// K1 and then N2 x K2 per slot whose x has at most x_rows rows: 16 or 32 for the walk,
+// kMoeTileRows for the tiles.
+int moe_walk_window(int64_t S, int64_t E);
+int moe_window(int64_t S, int64_t E, int64_t N1, int64_t K1, int64_t N2, int64_t K2,
+               int64_t x_rows, int bits, int group_size);
 int64_t moe_max_segments(int64_t S, int64_t E, int window);
 hipError_t launch_moe_qmvs(const MoeArgs& a, int nmat, int window, int64_t max_seg,
                            hipStream_t stream);
@@ -295,6 +315,11 @@ hipError_t launch_moe_qmvw_q4(const MoeArgs& a, int nmat, int window, int ntt, i
                               hipStream_t stream);
 hipError_t launch_moe_qmvw_q8(const MoeArgs& a, int nmat, int window, int ntt, int64_t max_seg,
                               hipStream_t stream);
+
+// The 64-slot tiles of longer expert runs (fmxq_moe_tile.hpp): a segment table cut
+// every kMoeTileRows slots.
+hipError_t launch_moe_tile_q4(const MoeArgs& a, int nmat, int64_t max_seg, hipStream_t stream);
+hipError_t launch_moe_tile_q8(const MoeArgs& a, int nmat, int64_t max_seg, hipStream_t stream);
 
 // Few-slot down projection fused with the top-k combine (one block per row
 // tile and token, one wave per slot): out [T, D] from the h rows [T k, I].

@@ -626,7 +626,31 @@ bool moe_qmvs_supported(int64_t N, int64_t K, int64_t x_rows, int bits, int grou
 // 16-slot windows everywhere, configuration 4 at M=256 1699 -> 1825 us and
 // configuration 3 at M=512 346 -> 365 us; 32-slot windows everywhere,
 // configuration 3 at M=16 79 -> 83 us.
-int moe_window(int64_t S, int64_t E) { return S >= 4 * E ? 32 : 16; }
+int moe_walk_window(int64_t S, int64_t E) { return S >= 4 * E ? 32 : 16; }
+
+// The tiles (fmxq_moe_tile.hpp) from 16 slots per expert, where the batch also fills
+// the chip with their larger blocks: 4096 slots, or 48 per expert and about two
+// blocks per CU in the first product.  A layer with the
+// router and shared expert, walk against tiles (us): 512 experts x 512, K = 2048,
+// top-10: 700 tokens (14 slots per expert) 290 / 297, 820 (16) 352 / 310, 2000 (39)
+// 632 / 411; 256 experts x 2048, K = 7168, top-8: 450 tokens (16) 1793 / 1675, 1024
+// (36) 2705 / 2189; 64 experts x 1536, K = 3072, top-6: 250 tokens (23, 1500 slots)
+// 186 / 196, 600 (56) 340 / 254, 900 (84) in groups of 32 688 / 498; 16 experts x 1792,
+// top-8, 1407 tokens (703) 1021 / 662; 16 experts x 1024, K = 2048, top-4: 200 tokens
+// (50, 264 blocks) 69 / 72.  Batches the tiles do not take (outputs not a multiple of
+// 32, x of 2^31 bytes, the allocation-free call's scratch) keep the walk and, for their
+// long runs, the grouped GEMM.
+int moe_window(int64_t S, int64_t E, int64_t N1, int64_t K1, int64_t N2, int64_t K2,
+               int64_t x_rows, int bits, int group_size) {
+  const int64_t kmax = K1 > K2 ? K1 : K2;
+  const int64_t blocks = (E + S / kMoeTileRows) * ((N1 + 127) / 128);
+  if (S >= 16 * E && (S >= 4096 || (S >= 48 * E && blocks >= 512)) && N1 % 32 == 0 && N2 % 32 == 0 &&
+      x_rows * kmax * 2 < (int64_t(1) << 31) &&
+      moe_qmvs_supported(N1, K1, x_rows, bits, group_size) &&
+      moe_qmvs_supported(N2, K2, x_rows, bits, group_size))
+    return kMoeTileRows;
+  return moe_walk_window(S, E);
+}
 
 int64_t moe_max_segments(int64_t S, int64_t E, int window) {
   const int64_t runs = S < E + 1 ? S : E + 1;
@@ -637,7 +661,7 @@ int64_t moe_max_segments(int64_t S, int64_t E, int window) {
 hipError_t launch_moe_qmvs(const MoeArgs& a, int nmat, int window, int64_t max_seg,
                            hipStream_t stream) {
   if (a.S <= 0 || a.N <= 0 || max_seg <= 0) return hipSuccess;
-  if (!moe_qmvs_supported(a.N, a.K, a.x_rows, a.bits, a.group_size) || (window != 16 && window != 32) ||
+  if (!moe_qmvs_supported(a.N, a.K, a.x_rows, a.bits, a.group_size) || (window != 16 && window != 32 && window != kMoeTileRows) ||
       (nmat != 1 && nmat != 2))
     return hipErrorInvalidValue;
   // Without a segment table (the few-slot path: every slot its own segment), rows
@@ -647,6 +671,11 @@ hipError_t launch_moe_qmvs(const MoeArgs& a, int nmat, int window, int64_t max_s
   // pair, and the walk measured as fast as a separate GEMV launch for those
   // segments or faster (configuration 3 at M=16 86 -> 81 us, at M=128 248 -> 239
   // us), without the GEMV grid's blocks for every other segment.
+  if (window == kMoeTileRows && a.seg) {
+    if (a.N % 32 || a.sh_T > 0 || !a.xprep || !moe_xlds_supported(a.x, a.x_rows, a.K)) return hipErrorInvalidValue;
+    return a.bits == 4 ? launch_moe_tile_q4(a, nmat, max_seg, stream)
+                       : launch_moe_tile_q8(a, nmat, max_seg, stream);
+  }
   MoeArgs b = a;
   const bool gemv = a.K >= 2048 && a.K <= 16384 && !a.seg;
   // Shared-expert segments exist in the GEMV form, without an output row map, and

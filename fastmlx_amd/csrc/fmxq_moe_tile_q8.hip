@@ -1,0 +1,15 @@
+// fmxq_moe_tile_q8.hip -- the 64-slot MoE tiles for 8-bit weights.
+#include "fmxq_moe_tile.hpp"
+
+namespace fmxq {
+
+hipError_t launch_moe_tile_q8(const MoeArgs& a, int nmat, int64_t max_seg, hipStream_t stream) {
+  switch (a.group_size) {
+    case 32: return launch_moe_tile_fmt<8, 32>(a, nmat, max_seg, stream);
+    case 64: return launch_moe_tile_fmt<8, 64>(a, nmat, max_seg, stream);
+    case 128: return launch_moe_tile_fmt<8, 128>(a, nmat, max_seg, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace fmxq

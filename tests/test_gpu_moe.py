@@ -844,6 +844,100 @@ def test_moe_layer_gated_shared_expert(gpu, oracle, T, E, D, k):
                          what=f"moe_layer gated T={T}")
 
 
+# --- the 64-slot tiles of longer expert runs (from 16 slots per expert on average, here in
+# --- batches of 4096 slots) ---
+
+# Edges of the 32-row halves and the 64-slot tiles, and a run that makes it a batch of
+# more than 4096 slots.
+TILE_RUNS = [1, 32, 33, 64, 65, 130, 3800]
+
+
+@pytest.mark.parametrize("bits,group", [(4, 32), (4, 64), (4, 128), (8, 32), (8, 64), (8, 128)])
+@pytest.mark.parametrize("D,I", [(256, 512), (768, 256), (2304, 1280)])
+def test_switch_glu_tiles(gpu, oracle, bits, group, D, I):
+    """Runs at the tile edges in every format: one step pair, an odd number of them, and
+    more than the scales of one load (the bounds of tests/parity.py against the
+    exact-affine oracle, which the tiles compute), with one bad id."""
+    from fastmlx_amd import FmxqError, ops
+
+    rng = np.random.default_rng(D + I + bits + group)
+    E, T = len(TILE_RUNS), sum(TILE_RUNS)
+    gate, up, down = _stack(rng, E, D, I, bits, group)
+    x = make_x(rng, T, D)
+    inds = rng.permutation(np.repeat(np.arange(E), TILE_RUNS))[:, None].astype(np.int32)
+    inds[7, 0] = E + 9
+    announce(f"switch_glu tiles {bits}-bit group {group} D={D} I={I}")
+    got = _run(gpu, x, inds, gate, up, down, group, bits)
+    with pytest.raises(FmxqError):
+        ops.device_error()
+    ok = inds < E
+    assert np.all(got[~ok] == 0)
+    sel = np.unique(np.concatenate([np.flatnonzero(inds[:, 0] == e)[[0, -1]] for e in range(E)]
+                                   + [rng.choice(T, 40, replace=False)]))
+    sel = sel[ok[sel, 0]]
+    sref = parity.SwitchRef(x, np.where(ok, inds, 0), gate, up, down, group, bits, token_sel=sel,
+                            fused=False)
+    parity.check_switch(got[sel], sref, what="tiles")
+
+
+@pytest.mark.parametrize("bits,group,N", [(4, 64, 160), (8, 64, 416), (4, 32, 32)])
+def test_gather_qmm_tiles(gpu, oracle, bits, group, N):
+    """Output widths that leave waves of a tile without columns, gathered x rows out of
+    order, and a bad x row (its output row is zero)."""
+    from fastmlx_amd import FmxqError, ops
+
+    rng = np.random.default_rng(N + bits)
+    E, K = len(TILE_RUNS), 1280
+    w, s, b = make_quant(rng, (E, N), K, bits, group)
+    rhs = np.repeat(np.arange(E), TILE_RUNS).astype(np.uint32)
+    lhs = rng.permutation(len(rhs)).astype(np.uint32)
+    lhs[100] = len(rhs) + 4
+    x = make_x(rng, len(rhs), 1, K)
+    dev = lambda t: to_dev(t, gpu)
+    announce(f"gather_qmm tiles {bits}-bit group {group} N={N}")
+    y = ops.gather_qmm(dev(x), dev(w), dev(s), dev(b), dev(rhs), dev(lhs), 1, True, group, bits, True)
+    torch.cuda.synchronize()
+    with pytest.raises(FmxqError):
+        ops.device_error()
+    got = to_np(y).reshape(-1, N)
+    ok = lhs < len(rhs)
+    assert np.all(got[~ok] == 0)
+    ref = parity.gather_refs(x.reshape(-1, K), w, s, b, lhs[ok].astype(np.int32),
+                             rhs[ok].astype(np.int32), group, bits)
+    parity.check_dense(got[ok], ref, what="gather_qmm tiles")
+
+
+def test_moe_layer_tiles_shared_expert(gpu, oracle):
+    """The shared expert sorted in with one slot per token, as a run of its own tiles, and
+    two calls in a row with the same bits (the sort may order a run either way; a row's
+    sum does not depend on its place)."""
+    from fastmlx_amd import ops
+
+    rng = np.random.default_rng(77)
+    E, T, k, D, I = 4, 1400, 2, 512, 256
+    gate, up, down = _stack(rng, E, D, I)
+    sh = _stack(rng, 1, D, I)
+    x = make_x(rng, T, D)
+    inds = topk_uniform(rng, T, E, k)
+    w16 = oracle.f32_to_bf16(rng.dirichlet(np.ones(k), size=T).astype(np.float32))
+    dev = lambda t: to_dev(t, gpu)
+    args = (dev(x), dev(inds.astype(np.uint32)), *[tuple(map(dev, m)) for m in (gate, up, down)],
+            dev(w16), [tuple(map(dev, m)) for m in sh])
+    announce("moe_layer tiles with the shared expert")
+    a, b = ops.moe_layer(*args), ops.moe_layer(*args)
+    torch.cuda.synchronize()
+    ops.device_error()
+    assert torch.equal(a, b)
+    sel = np.unique(np.concatenate([[0, T - 1], rng.choice(T, 60, replace=False)]))
+    sref = parity.SwitchRef(x, inds, gate, up, down, token_sel=sel, fused=False)
+    near = sref.refs[0]
+    ssref = parity.SwitchRef(x, np.zeros((T, 1), np.int32), *sh, token_sel=sel, fused=False)
+    sv = ssref.refs[0]
+    sa = parity.switch_bound(sv, sv, ssref.hscale)
+    parity.combine_check(to_np(a)[sel], near, parity.switch_bound(near, near, sref.hscale), w16[sel],
+                         shared=(sv[:, 0], sa[:, 0]), what="moe_layer tiles")
+
+
 # --- the weight formats other than 4 bits in groups of 64 ---
 
 @pytest.mark.parametrize("bits,group", [(4, 32), (4, 128), (8, 32), (8, 64), (8, 128)])
