@@ -2,17 +2,20 @@
 
 ``python -m fastmlx_amd.build`` or ``fastmlx_amd.build.build()``.  Objects go to
 ``fastmlx_amd/_build/``; the shared library lands next to this file so it
-travels with the source tree.  ``--diag`` (``build_diag()``) also builds the
+travels with the source tree, and so does ``_fast.so``, the torch wrappers' call path.
+``--diag`` (``build_diag()``) also builds the
 time-line diagnostic program ``diag/qmv1_timeline``.
 """
 from __future__ import annotations
 
 import concurrent.futures as cf
 import glob
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -70,6 +73,33 @@ def build_diag(verbose: bool = True) -> str:
     return TIMELINE
 
 
+FAST = os.path.join(HERE, "_fast.so")
+
+
+def build_fast(verbose: bool = True) -> str:
+    """The torch wrappers' call path in C++ (ext/fmxq_fast.cpp), a CPython module linked
+    against torch and the libfmxq.so next to it."""
+    torch_dir = list(importlib.util.find_spec("torch").submodule_search_locations)[0]
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    inc = [os.path.join(torch_dir, "include"), sysconfig.get_paths()["include"],
+           os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
+           os.path.join(rocm, "include")]
+    lib = os.path.join(torch_dir, "lib")
+    tmp = FAST + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", *(a for d in inc for a in ("-isystem", d)),
+           os.path.join(HERE, "ext", "fmxq_fast.cpp"), "-o", tmp, f"-L{lib}", "-lc10", "-lc10_hip",
+           "-ltorch_cpu", "-ltorch_python", f"-L{HERE}", "-l:libfmxq.so", "-Wl,-rpath,$ORIGIN",
+           f"-Wl,-rpath,{lib}"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"compile failed: {' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, FAST)
+    if verbose:
+        print(f"built {FAST}")
+    return FAST
+
+
 def build(verbose: bool = True) -> str:
     os.makedirs(OUT_DIR, exist_ok=True)
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")) + glob.glob(os.path.join(CSRC, "*.cpp")))
@@ -86,6 +116,7 @@ def build(verbose: bool = True) -> str:
     os.replace(tmp, LIB)
     if verbose:
         print(f"built {LIB}")
+    build_fast(verbose)
     return LIB
 
 

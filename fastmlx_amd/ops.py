@@ -11,6 +11,13 @@ import torch
 
 from ._lib import check, load
 
+try:
+    # The same calls checked and launched from C++ (ext/fmxq_fast.cpp): a function
+    # returns None for anything out of the ordinary, and the Python path below takes it.
+    from . import _fast
+except ImportError:  # not built: every call takes the Python path
+    _fast = None
+
 _BF16_LIKE = (torch.bfloat16, torch.int16, torch.uint16)
 _U32_LIKE = (torch.int32, torch.uint32)
 
@@ -33,6 +40,10 @@ def _stream(t: torch.Tensor) -> int:
 
 def dequantize(w, scales, biases, group_size: int = 64, bits: int = 4, out=None):
     """MLX dequantize: [..., K*bits/32] packed -> [..., K] bf16."""
+    if _fast is not None:
+        y = _fast.dequantize(w, scales, biases, out, group_size, bits)
+        if y is not None:
+            return y
     K = w.shape[-1] * 32 // bits
     rows = w.numel() // max(w.shape[-1], 1)
     if out is None:
@@ -47,6 +58,10 @@ def quantize(w, group_size: int = 64, bits: int = 4, out=None):
     """MLX affine quantize: bf16 [..., K] -> (packed [..., K*bits/32] int32 words,
     scales [..., K/group] bf16, biases [..., K/group] bf16); ``out`` may hold the
     three result tensors."""
+    if _fast is not None and out is None:
+        q = _fast.quantize(w, group_size, bits)
+        if q is not None:
+            return q
     K = w.shape[-1]
     rows = w.numel() // max(K, 1)
     if K % group_size:
@@ -68,6 +83,10 @@ def quantize(w, group_size: int = 64, bits: int = 4, out=None):
 def quantized_matmul(x, w, scales, biases, transpose: bool = True, group_size: int = 64,
                      bits: int = 4, bias=None, out=None):
     """y = x @ deq(W)^T over x [..., K]; W [N, K*bits/32]; y [..., N] bf16."""
+    if _fast is not None and transpose is True:
+        y = _fast.quantized_matmul(x, w, scales, biases, bias, out, group_size, bits)
+        if y is not None:
+            return y
     K = x.shape[-1]
     N = w.shape[0]
     M = x.numel() // max(K, 1)
@@ -165,6 +184,11 @@ def switch_glu_combine(x, inds, gate, up, down, weights, shared=None, shared_gat
 
     weights [T, top_k] bf16; shared [T, D] (optional) is added, sigmoid-gated by
     shared_gate [T] when given.  Returns [T, D] bf16."""
+    if _fast is not None:
+        y = _fast.moe_layer(x, inds, gate, up, down, weights, None, shared, shared_gate, out,
+                            group_size, bits)
+        if y is not None:
+            return y
     T, D = x.shape
     topk = inds.shape[-1]
     E, I = gate[0].shape[0], gate[0].shape[1]
@@ -188,6 +212,11 @@ def moe_layer(x, inds, gate, up, down, weights, shared_expert, shared_gate=None,
 
     shared_expert = (gate, up, down) triples of a one-expert stack; shared_gate [T]
     (optional) sigmoid-gates its output.  Returns [T, D] bf16."""
+    if _fast is not None and shared_expert is not None:
+        y = _fast.moe_layer(x, inds, gate, up, down, weights, shared_expert, None, shared_gate, out,
+                            group_size, bits)
+        if y is not None:
+            return y
     T, D = x.shape
     topk = inds.shape[-1]
     E, I = gate[0].shape[0], gate[0].shape[1]
@@ -232,6 +261,11 @@ def _route_io(logits, T, k, weights_dtype):
 def route_softmax_topk(logits, top_k, norm_topk_prob=True, weights_dtype=torch.bfloat16):
     """Softmax router (qwen3next_forward.go:513-518): logits [T, E] -> (inds [T, k] int32
     holding uint32 ids, weights [T, k]), largest gate first."""
+    if _fast is not None and weights_dtype in (torch.bfloat16, torch.float32):
+        r = _fast.route_softmax_topk(logits, top_k, bool(norm_topk_prob),
+                                     weights_dtype is torch.bfloat16)
+        if r is not None:
+            return r
     T, E = logits.shape
     inds, weights = _route_io(logits, T, top_k, weights_dtype)
     ptr = _dev(logits, "logits", (torch.bfloat16, torch.float32))
@@ -246,6 +280,12 @@ def route_group_topk(gates, bias, top_k, n_group, topk_group, routed_scaling_fac
                      norm_topk_prob=True, weights_dtype=torch.float32):
     """DeepSeek-V3 group-limited router (deepseekv3_forward.go:452-491): gates [T, E],
     bias [E] float32 or None -> (inds [T, k] int32 holding uint32 ids, weights [T, k])."""
+    if _fast is not None and weights_dtype in (torch.bfloat16, torch.float32):
+        r = _fast.route_group_topk(gates, bias, top_k, n_group, topk_group,
+                                   float(routed_scaling_factor), bool(norm_topk_prob),
+                                   weights_dtype is torch.bfloat16)
+        if r is not None:
+            return r
     T, E = gates.shape
     inds, weights = _route_io(gates, T, top_k, weights_dtype)
     bptr = None if bias is None else _dev(bias, "bias", (torch.float32,))
