@@ -322,7 +322,10 @@ int qmm_common(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
   // stays); 4096x4096 M = 8 13.0 -> 9.3 (M = 5 9.4 against 9.3 stays); narrower
   // outputs keep the GEMV up to M = 8: 1024x4096 M = 8 5.8 against 6.9) and the
   // prefill GEMM's 64-row tile (M = 9-16 on 4096x4096 16.5-17.3 -> 9.4-9.6).
-  const bool walk4 = bits == 4 && M > 8 && (M > 16 || N >= 8192 || K >= 8192);
+  // int4 in groups of 32 or 128: from M = 5 (qmvs has groups of 64 only; against the
+  // prefill GEMM's 64-row tile: 1024x4096 13.3 -> 8.3 us, 14336x4096 34.0 -> 15.3).
+  const bool walk4 = bits == 4 && (group_size == 64 ? M > 8 && (M > 16 || N >= 8192 || K >= 8192)
+                                                    : M > 4);
   const bool walk8 = bits == 8 && (M >= 9 || (M >= 2 && K >= 8192) || (M >= 3 && N >= 8192) ||
                                    (M >= 8 && N >= 4096));
   if ((walk4 || walk8) && M <= fmxq::kQmvwMaxM && fmxq::qmvw_supported(a)) {

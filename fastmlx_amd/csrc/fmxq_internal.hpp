@@ -106,7 +106,7 @@ bool qmvs_supported(const QmmArgs& a);
 hipError_t launch_qmvs(const QmmArgs& a, hipStream_t stream);
 bool qmv_mfma_supported(const QmmArgs& a);
 hipError_t launch_qmv_mfma(const QmmArgs& a, hipStream_t stream);
-// int4 / int8 group-64 product for M <= kQmvwMaxM with x shared through LDS by the waves
+// int4 / int8 product for M <= kQmvwMaxM with x shared through LDS by the waves
 // of a block and K split over blocks (fmxq_skinny.hip, qmvw_kernel).
 constexpr int kQmvwMaxM = 64;
 struct QmvwPlan {
@@ -116,6 +116,9 @@ struct QmvwPlan {
 bool qmvw_supported(const QmmArgs& a);
 QmvwPlan qmvw_plan(const QmmArgs& a, int cus);
 hipError_t launch_qmvw(const QmmArgs& a, const QmvwPlan& p, hipStream_t stream);
+// Its kernels for groups of 32 and 128 (fmxq_qmvw_fmt.hip).
+hipError_t launch_qmvw_fmt(const QmmArgs& a, const QmvwPlan& p, hipStream_t stream);
+constexpr int kQmvwMaxParts = 16;
 
 // MFMA GEMM for larger M.  qmm_plan() reports the split-K factor and the
 // workspace launch_qmm() will need for these sizes.

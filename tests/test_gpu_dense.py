@@ -290,6 +290,25 @@ def test_qmvw_int8(gpu, oracle, M, N, K, bias):
     assert np.array_equal(r1, r2)
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("group", [32, 128])
+@pytest.mark.parametrize("M,N,K,bias", [
+    (5, 72, 256, False),      # one step, a part-full W tile
+    (9, 1000, 1792, True),    # narrow: up-front pairs of steps in parts (4 bits), odd steps
+    (16, 4096, 1024, False),  # up-front walk of a whole part
+    (17, 8200, 768, True),    # 32-row W tiles (4 bits), ragged
+    (32, 512, 8448, False),   # long rows: pipelined parts of unequal length
+    (33, 4100, 512, False),   # 64 x rows, 4-wave blocks up front or 8-wave pipelined
+    (64, 8192, 2304, True),   # 64 x rows, wide
+])
+def test_qmvw_formats(gpu, oracle, bits, group, M, N, K, bias):
+    """The shared-x walk in groups of 32 and 128, on every plan branch (test_qmvw_*
+    cover groups of 64)."""
+    rows = np.unique(np.array([0, 1, M // 2, M - 2, M - 1]))
+    _qmm_case(gpu, oracle, M, N, K, bits, group, seed=9700 + M + N + K + group, rows_checked=rows,
+              bias=bias)
+
+
 @pytest.mark.parametrize("M,N,K,bits,group", [
     (384, 1024, 1024, 4, 64),    # the threshold M
     (383, 1024, 1024, 4, 64),    # one row below it: the prefill GEMM
