@@ -1,6 +1,9 @@
 // fmxq_qmm_wide.hip -- MFMA GEMM with the dequantization in registers, for
 // quantized_matmul at prefill sizes (qmm_use_wide: M >= 384 rows of x, or
-// M >= 128 for outputs at least twice the depth).
+// M >= 128 for outputs at least twice the depth), in groups of 32, 64 and 128.  (Groups
+// of 32 and 128 ran the prefill GEMM: 4096x14336 at M = 2048 in groups of 32 258 -> 216
+// us, 23552x11008 at M = 331 in groups of 128 299 -> 231 us, 8 bits in groups of 32
+// 8192x4096 at M = 2000 153 -> 124 us.)
 //
 // Replaces the GEMM of mlx_quantized_matmul (mlxgo/binding_cgo.go:636-643) for
 // x [M, K] with M = batch * seq rows: prefill through compute/models/quant.go:91-101
@@ -71,7 +74,7 @@ struct WideCfg {
 
 enum Role { kFull = 0, kContrib = 1, kFinal = 2 };
 
-template <int BITS, int WAVES, int BM>
+template <int BITS, int WAVES, int BM, int GS>
 __global__ __launch_bounds__(WAVES * 64, 1) void qmm_wide_kernel(WideArgs wa) {
   using C = WideCfg<BITS, WAVES, BM>;
   static_assert(WAVES == 8, "the output staging gives each of 8 waves 4 rows of a 32-row group");
@@ -95,7 +98,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void qmm_wide_kernel(WideArgs wa) {
   const int wcol = 32 * JT * wave;                      // first output of this wave in the tile
 
   const int64_t wpr = a.K * BITS / 32;                 // packed words per weight row
-  const int64_t gpr = a.K / kS;                        // groups (of 64) per row
+  const int64_t gpr = a.K / GS;                        // groups per row
   const __amdgpu_buffer_rsrc_t wres = __builtin_amdgcn_make_buffer_rsrc(
       (void*)a.w, (short)0, (int)(a.N * wpr * 4), 0x00020000);
   const __amdgpu_buffer_rsrc_t sres = __builtin_amdgcn_make_buffer_rsrc(
@@ -121,11 +124,13 @@ __global__ __launch_bounds__(WAVES * 64, 1) void qmm_wide_kernel(WideArgs wa) {
   bf16x8 af0[JT][4], af1[JT][4];   // A operands of two consecutive steps
   bf16x8 xf0[RT], xf1[RT];         // B operands of two consecutive sub-steps
   u32x4 wq[4][JT][NLD];            // packed weights, one set per step in flight
-  // Scales and biases of four steps (one group each), words {s(0,1), s(2,3),
-  // b(0,1), b(2,3)}: lane L holds those of weight row wcol + L (JT = 2) or of
-  // row wcol + L % 32 (JT = 1).  sbA serves the current four steps, sbB is loaded
-  // for the next four.
-  uint32_t sbA[4], sbB[4];
+  // Scales and biases of four steps (256 values: 8, 4 or 2 groups), SW words of scale
+  // pairs, then SW of bias pairs: lane L holds those of weight row wcol + L (JT = 2)
+  // or of row wcol + L % 32 (JT = 1).  sbA serves the current four steps, sbB is
+  // loaded for the next four.
+  constexpr int SW = 128 / GS;
+  static_assert(SW == 1 || SW == 2 || SW == 4, "group size");
+  uint32_t sbA[2 * SW], sbB[2 * SW];
 
   // Work items of this block: dp whole tiles (dealt to the XCDs so that each
   // one's resident blocks hold neighbouring tiles), then the stream-K pieces.
@@ -172,16 +177,25 @@ __global__ __launch_bounds__(WAVES * 64, 1) void qmm_wide_kernel(WideArgs wa) {
     int64_t n_sb = n0 + wcol + (JT == 2 ? lane : r32);
     if (n_sb > a.N - 1) n_sb = a.N - 1;
     const uint32_t sbo = (uint32_t)(n_sb * gpr * 2);
-    // Scales and biases of steps k .. k + 3 (8-byte aligned: gpr and k are
-    // multiples of 4).
-    auto load_sb = [&](uint32_t (&sb)[4], int k) {
+    // Scales and biases of steps k .. k + 3 (aligned to their 4 SW bytes: gpr and the
+    // step's group are multiples of 2 SW).
+    auto load_sb = [&](uint32_t (&sb)[2 * SW], int k) {
       k = k < ke - 4 ? k : ke - 4;
-      const u32x2 sv = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(sres, (int)sbo, k * 2, 0));
-      const u32x2 bv = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(bres, (int)sbo, k * 2, 0));
-      sb[0] = sv[0];
-      sb[1] = sv[1];
-      sb[2] = bv[0];
-      sb[3] = bv[1];
+      const int off = k * (kS * 2) / GS;  // 2 bytes a group
+      if constexpr (SW == 1) {
+        sb[0] = __builtin_amdgcn_raw_buffer_load_b32(sres, (int)sbo, off, 0);
+        sb[1] = __builtin_amdgcn_raw_buffer_load_b32(bres, (int)sbo, off, 0);
+      } else if constexpr (SW == 2) {
+        const u32x2 sv = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(sres, (int)sbo, off, 0));
+        const u32x2 bv = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(bres, (int)sbo, off, 0));
+#pragma unroll
+        for (int i = 0; i < 2; ++i) sb[i] = sv[i], sb[2 + i] = bv[i];
+      } else {
+        const u32x4 sv = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(sres, (int)sbo, off, 0));
+        const u32x4 bv = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(bres, (int)sbo, off, 0));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) sb[i] = sv[i], sb[4 + i] = bv[i];
+      }
     };
 
     // Loads of step k: the packed weights first, then the x DMA, so a wait for
@@ -205,16 +219,18 @@ __global__ __launch_bounds__(WAVES * 64, 1) void qmm_wide_kernel(WideArgs wa) {
             xres, (lds_t*)(stage(st) + 8 * (XI * wave + i) * 128), 16, (int)xdo[i], xoff, 0, 0);
     };
     // The scale and bias of step offset o (0..3) of sb as fp32 for each row group
-    // of the lane.  With two row groups lane L holds row L's, and
+    // of the lane.  (Groups of 32: a lane half's four chunks of a step are one group.)  With two row groups lane L holds row L's, and
     // v_permlane32_swap on two copies gives rows 0..31 to both halves of the wave
     // (row group 0) and rows 32..63 to both halves (row group 1).
     struct SB {
       float s[JT], b[JT];
     };
-    auto scale_bias = [&](const uint32_t (&sb)[4], int o) {
-      const uint32_t sw = sb[o >> 1], bw = sb[2 + (o >> 1)];
-      const uint32_t sf = (o & 1) ? (sw & 0xffff0000u) : (sw << 16);
-      const uint32_t bf = (o & 1) ? (bw & 0xffff0000u) : (bw << 16);
+    auto scale_bias = [&](const uint32_t (&sb)[2 * SW], int o) {
+      const int word = GS == 32 ? o : GS == 64 ? o >> 1 : 0;
+      const bool hi = GS == 32 ? h != 0 : GS == 64 ? (o & 1) != 0 : o >= 2;
+      const uint32_t sw = sb[word], bw = sb[SW + word];
+      const uint32_t sf = hi ? (sw & 0xffff0000u) : (sw << 16);
+      const uint32_t bf = hi ? (bw & 0xffff0000u) : (bw << 16);
       SB r;
       if constexpr (JT == 2) {
         const auto sp = __builtin_amdgcn_permlane32_swap(sf, sf, false, false);
@@ -339,7 +355,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void qmm_wide_kernel(WideArgs wa) {
       step(k + 2, std::integral_constant<int, 2>{}, tc, af0, af1);
       step(k + 3, std::integral_constant<int, 3>{}, tc, af1, af0);
 #pragma unroll
-      for (int q = 0; q < 4; ++q) sbA[q] = sbB[q];
+      for (int q = 0; q < 2 * SW; ++q) sbA[q] = sbB[q];
     };
     int k = kb;
     for (; k + 4 < ke; k += 4) pass(k, std::false_type{});
@@ -462,6 +478,20 @@ __global__ __launch_bounds__(WAVES * 64, 1) void qmm_wide_kernel(WideArgs wa) {
   }
 }
 
+template <int GS>
+hipError_t launch_wide_gs(const WideArgs& wa, const WidePlan& p, hipStream_t stream) {
+  constexpr int W = kWideWaves;
+  const dim3 grid((unsigned)p.blocks), block(W * 64);
+  if (p.bm == 256) {
+    if (wa.q.bits == 4) qmm_wide_kernel<4, W, 256, GS><<<grid, block, 0, stream>>>(wa);
+    else qmm_wide_kernel<8, W, 256, GS><<<grid, block, 0, stream>>>(wa);
+  } else {
+    if (wa.q.bits == 4) qmm_wide_kernel<4, W, 128, GS><<<grid, block, 0, stream>>>(wa);
+    else qmm_wide_kernel<8, W, 128, GS><<<grid, block, 0, stream>>>(wa);
+  }
+  return hipGetLastError();
+}
+
 }  // namespace
 
 WidePlan qmm_wide_plan(int64_t M, int64_t N, int64_t K, int cus) {
@@ -511,7 +541,8 @@ bool qmm_wide_supported(const QmmArgs& a) {
   return a.M >= 1 && a.N >= 1 && a.K % (4 * kS) == 0 && a.K > 0 && a.ldx % 8 == 0 &&
          // 16-byte output stores of 8 outputs
          a.N % 8 == 0 && a.ldy % 8 == 0 && (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 &&
-         (a.bits == 4 || a.bits == 8) && a.group_size == kS && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 &&
+         (a.bits == 4 || a.bits == 8) &&
+         (a.group_size == 32 || a.group_size == 64 || a.group_size == 128) && (reinterpret_cast<uintptr_t>(a.x) & 15) == 0 &&
          (reinterpret_cast<uintptr_t>(a.w) & 15) == 0 &&
          // buffer resources count bytes in 32 bits: x per tile, w / scales / biases whole
          kT * a.ldx * 2 < ((int64_t)1 << 31) && a.N * (a.K * a.bits / 8) < ((int64_t)1 << 31) &&
@@ -523,16 +554,11 @@ hipError_t launch_qmm_wide(const QmmArgs& a, const WidePlan& p, uint32_t* err, h
     return hipErrorInvalidValue;
   if (p.sk_len > 0 && (!a.ws || !a.tile_count || !err)) return hipErrorInvalidValue;
   WideArgs wa{a, p.tm, p.nk, p.dp, p.sk_len, p.sk_iters, err};
-  constexpr int W = kWideWaves;
-  const dim3 grid((unsigned)p.blocks), block(W * 64);
-  if (p.bm == 256) {
-    if (a.bits == 4) qmm_wide_kernel<4, W, 256><<<grid, block, 0, stream>>>(wa);
-    else qmm_wide_kernel<8, W, 256><<<grid, block, 0, stream>>>(wa);
-  } else {
-    if (a.bits == 4) qmm_wide_kernel<4, W, 128><<<grid, block, 0, stream>>>(wa);
-    else qmm_wide_kernel<8, W, 128><<<grid, block, 0, stream>>>(wa);
+  switch (a.group_size) {
+    case 32: return launch_wide_gs<32>(wa, p, stream);
+    case 64: return launch_wide_gs<64>(wa, p, stream);
+    default: return launch_wide_gs<128>(wa, p, stream);
   }
-  return hipGetLastError();
 }
 
 }  // namespace fmxq

@@ -293,6 +293,22 @@ def test_qmvw_int8(gpu, oracle, M, N, K, bias):
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("group", [32, 128])
 @pytest.mark.parametrize("M,N,K,bias", [
+    (384, 264, 256, False),   # one pass of four steps, a part-full output tile
+    (130, 2056, 1024, True),  # wide outputs from M = 128, 128-row tiles, stream-K pieces
+    (513, 768, 2304, True),   # an odd number of passes, one x row in the last tile
+    (2050, 8200, 768, False), # 256-row tiles, whole tiles and stream-K
+])
+def test_qmm_wide_formats(gpu, oracle, bits, group, M, N, K, bias):
+    """The wide GEMM in groups of 32 and 128 (a lane half's scales and four steps' scales
+    in one word), on both tile heights."""
+    rows = np.unique(np.array([0, 1, 127, M // 2, M - 2, M - 1]))
+    _qmm_case(gpu, oracle, M, N, K, bits, group, seed=9800 + M + N + K + group, rows_checked=rows,
+              bias=bias)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("group", [32, 128])
+@pytest.mark.parametrize("M,N,K,bias", [
     (5, 72, 256, False),      # one step, a part-full W tile
     (9, 1000, 1792, True),    # narrow: up-front pairs of steps in parts (4 bits), odd steps
     (16, 4096, 1024, False),  # up-front walk of a whole part
