@@ -30,8 +30,6 @@
 // group scores use 64 / n_group lanes for each group at once instead of a
 // wave-wide reduction per group.  Measured (rocprof medians): E = 512, k = 10 softmax
 // at T = 1 10.8 -> 6.6 us; E = 256, k = 8 of 4 of 8 groups at T = 1024 15.6 -> 8.1 us.
-#include <type_traits>
-
 #include "fmxq_common.hpp"
 #include "fmxq_internal.hpp"
 
@@ -45,8 +43,8 @@ __device__ __forceinline__ uint32_t dpp_or(uint32_t old, uint32_t v) {
   return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, RMASK, 0xf, false);
 }
 
-// Wave-wide reductions on DPP: quad swaps, half-row and row mirrors, then the row
-// broadcasts, which leave the total in lane 63.
+// The wave's maximum on DPP: quad swaps, half-row and row mirrors, then the row
+// broadcasts, which leave it in lane 63.
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   v = max(v, dpp_or<0xb1, 0xf>(0, v));
   v = max(v, dpp_or<0x4e, 0xf>(0, v));
@@ -57,18 +55,20 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
   return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
+// The wave's sum in every lane, added as __shfl_xor by 32, 16, .. 1 adds it (wave_sum),
+// so that the weights do not depend on how the lanes are read: half and row swaps for
+// the first two steps, then DPP.  After the step of distance d a lane's value depends on
+// its number mod d only, so a rotation within the row of 16 reads the same value as xor.
 __device__ __forceinline__ float wave_add(float v) {
-  auto step = [&](auto ctrl, auto rmask) {
-    v += __uint_as_float(dpp_or<decltype(ctrl)::value, decltype(rmask)::value>(0, __float_as_uint(v)));
-  };
-  using std::integral_constant;
-  step(integral_constant<int, 0xb1>{}, integral_constant<int, 0xf>{});
-  step(integral_constant<int, 0x4e>{}, integral_constant<int, 0xf>{});
-  step(integral_constant<int, 0x141>{}, integral_constant<int, 0xf>{});
-  step(integral_constant<int, 0x140>{}, integral_constant<int, 0xf>{});
-  step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});
-  step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});
-  return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), 63));
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  v += __uint_as_float(dpp_or<0x128, 0xf>(0, __float_as_uint(v)));  // row_ror:8
+  v += __uint_as_float(dpp_or<0x124, 0xf>(0, __float_as_uint(v)));  // row_ror:4
+  v += __uint_as_float(dpp_or<0x4e, 0xf>(0, __float_as_uint(v)));   // quad_perm [2,3,0,1]
+  v += __uint_as_float(dpp_or<0xb1, 0xf>(0, __float_as_uint(v)));   // quad_perm [1,0,3,2]
+  return v;
 }
 
 // Order-preserving key: a < b as floats exactly when key(a) < key(b), -0 equal to

@@ -178,3 +178,55 @@ def test_router_feeds_switch_glu_combine(gpu, oracle):
     ref = (y.float() * w.float()[:, :, None]).sum(dim=1)
     assert torch.allclose(out.float(), ref, rtol=2e-2, atol=2e-2)
     assert (inds >= 0).all() and (inds < E).all()
+
+
+def _butterfly(lanes):
+    """fp32 sum of 64 lanes in the order of xor steps 32, 16, .. 1."""
+    v = lanes.astype(np.float32)
+    for off in (32, 16, 8, 4, 2, 1):
+        v = v + v[..., np.arange(64) ^ off]
+    return v[..., 0]
+
+
+@pytest.mark.parametrize("E", [64, 512])
+def test_softmax_denominator_order(gpu, E):
+    """The softmax denominator adds the lanes as xor steps 32, 16, .. 1.  Three experts
+    count in each row: 1 in lane 2^q and e = 0.75 * 2^-24 in lanes 0 and 2^p, the others
+    exactly 0.  1 + e rounds to 1 and 1 + 2 e to 1 + 2^-23, so the sum shows which of the
+    two steps came first."""
+    from fastmlx_amd import ops
+
+    announce(f"softmax denominator order E={E}")
+    pq = [(p, q) for p in range(6) for q in range(6) if p != q]
+    x = torch.full((len(pq), E), float("-inf"))
+    for t, (p, q) in enumerate(pq):
+        x[t, 2 ** q] = 0.0
+        x[t, 0] = x[t, 2 ** p] = float(np.log(0.75 * 2.0 ** -24))
+    inds, w = ops.route_softmax_topk(x.to(gpu), 1, False, torch.float32)
+    torch.cuda.synchronize()
+    w = w.cpu().numpy()[:, 0]
+    for t, (p, q) in enumerate(pq):
+        s = np.float32(1 + 2.0 ** -23) if p > q else np.float32(1)
+        assert int(inds[t, 0]) == 2 ** q
+        assert w[t] == np.float32(1) / s, (p, q, w[t])
+
+
+@pytest.mark.parametrize("T,E,k", [(37, 512, 10), (37, 64, 8), (9, 1024, 64)])
+def test_renormalization_order(gpu, T, E, k):
+    """The picked weights are divided by their sum over lanes 0 .. k - 1, added as xor
+    steps 32, 16, .. 1, in fp32: exact bits from the weights before the division."""
+    from fastmlx_amd import ops
+
+    announce(f"renormalization order T={T} E={E} k={k}")
+    g = torch.Generator().manual_seed(T + E + k)
+    x = torch.randn(T, E, generator=g).to(gpu)
+    for route in (lambda norm: ops.route_softmax_topk(x, k, norm, torch.float32),
+                  lambda norm: ops.route_group_topk(x, None, k, 8, 8, 1.0, norm, torch.float32)):
+        i0, w0 = route(False)
+        i1, w1 = route(True)
+        torch.cuda.synchronize()
+        assert torch.equal(i0, i1)
+        w0, w1 = w0.cpu().numpy(), w1.cpu().numpy()
+        lanes = np.zeros((T, 64), dtype=np.float32)
+        lanes[:, :k] = w0
+        assert np.array_equal(w1, w0 / _butterfly(lanes)[:, None])
