@@ -96,6 +96,30 @@ __device__ __forceinline__ bf16x8 cvt_frag8(uint32_t w0, uint32_t w1) {
                    pack_bf16x2((float)((w1 >> 16) & 0xffu), (float)(w1 >> 24)));
 }
 
+// x . w over values [k0, k1) of one weight row, the weights dequantized to bf16 as by
+// deq_frag4 / deq_frag8.  The affine forms (sum x (OFF + q) scaled, plus the bias term)
+// meet infinities of opposite sign where x holds one, or where their sums leave the fp32
+// range near x's largest values: an output that comes out infinite or NaN is taken again
+// in this form.  One lane, a value at a time: only such outputs pay for it, and a NaN ends
+// the walk.
+template <int BITS, int GS>
+__device__ inline float deq_row_dot(const uint16_t* x, const uint32_t* w, const uint16_t* sc,
+                                    const uint16_t* bi, int64_t k0, int64_t k1) {
+  constexpr int V = 32 / BITS;  // values per word
+  float t = 0.f;
+#pragma clang loop unroll(disable)
+  for (int64_t k = k0; k < k1 && t == t; k += V) {
+    const uint32_t q = w[k / V];
+    const float s = bf16_bits_to_f32(sc[k / GS]), b = bf16_bits_to_f32(bi[k / GS]);
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const float v = __builtin_fmaf(s, (float)((q >> (BITS * i)) & ((1u << BITS) - 1u)), b);
+      t = __builtin_fmaf(bf16_bits_to_f32(f32_to_bf16_rne(v)), bf16_bits_to_f32(x[k + i]), t);
+    }
+  }
+  return t;
+}
+
 // Exponent-trick offset per value and the factor that turns the ones-MFMA sum of
 // the A operand back into sum x (int8 A carries every x value twice).
 template <int BITS>

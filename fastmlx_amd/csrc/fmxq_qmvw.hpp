@@ -32,6 +32,8 @@ constexpr int kQmvwXallDeqMinMT = FMXQ_QMVW_XALL_DEQ_MIN_MT;
 // int8 weights in groups of 64 always take the dequantizing walks.  Groups of 32 and
 // 128 keep the exact affine form for one x tile (at 8 bits and few rows they came from
 // the exact dot2 GEMV) and dequantize from two, as the prefill GEMM they came from does.
+// That GEMM also answers rows of x with infinities, so the affine form takes its
+// non-finite outputs again, dequantized (deq_row_dot, over the block's own K part).
 template <int MT, int NTT, int WV, int D, int BITS, int GS>
 __global__ __launch_bounds__(WV * 64) __attribute__((amdgpu_waves_per_eu(MT == 1 && NTT == 1 && !(BITS == 8 && GS == 32) ? 3 : 2)))
 void qmvw_kernel(QmmArgs a) {
@@ -85,6 +87,13 @@ void qmvw_kernel(QmmArgs a) {
 
   // C layout of a 16x16 tile: register r of lane l is row 4 (l / 16) + r, column
   // l % 16.
+  constexpr bool kRedo = GS != 64 && !(D > 0 ? kDeqXall : kDeqXlds);
+  static_assert(!kRedo || NTT * MT * 4 <= 32, "one bit per output of a lane");
+  uint32_t odd = 0;
+  auto put = [&](int64_t m, int64_t n, float v) {
+    if (parts == 1) a.y[m * a.ldy + n] = finish_out(v, a.bias, n);
+    else a.ws[((int64_t)part * a.M + m) * a.N + n] = v;
+  };
 #pragma unroll
   for (int t = 0; t < NTT; ++t) {
     const int64_t n = nb + 16 * t + c16;
@@ -95,9 +104,19 @@ void qmvw_kernel(QmmArgs a) {
       for (int r = 0; r < 4; ++r) {
         const int64_t m = 16 * mt + 4 * q + r;
         if (m >= a.M) continue;
-        if (parts == 1) a.y[m * a.ldy + n] = finish_out(acc[0][mt][t][r], a.bias, n);
-        else a.ws[((int64_t)part * a.M + m) * a.N + n] = acc[0][mt][t][r];
+        const float v = acc[0][mt][t][r];
+        if constexpr (kRedo) odd |= __builtin_isfinite(v) ? 0u : 1u << ((t * MT + mt) * 4 + r);
+        put(m, n, v);
       }
+  }
+  if constexpr (kRedo) {
+    while (odd) {
+      const int i = __builtin_ctz(odd);
+      odd &= odd - 1;
+      const int64_t m = 16 * ((i >> 2) % MT) + 4 * q + (i & 3), n = nb + 16 * ((i >> 2) / MT) + c16;
+      put(m, n, deq_row_dot<BITS, GS>(a.x + m * a.ldx, a.w + n * (a.K * BITS / 32), a.scales + n * (a.K / GS),
+                                      a.biases + n * (a.K / GS), s0 * 256, s1 * 256));
+    }
   }
 }
 

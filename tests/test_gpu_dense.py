@@ -600,3 +600,58 @@ def test_quantized_matmul_group_graph_replay(gpu):
             assert np.array_equal(to_np(y), e), f"replay {rep} differs from eager"
         step()
         torch.cuda.synchronize()
+
+
+def _nonfinite_x(rng, M, K):
+    """M >= 5 rows of x: an infinity of either sign, a NaN, both infinities, and values near
+    the largest, in rows 0 to 4; the others ordinary."""
+    from oracle import f32_to_bf16
+
+    x = make_x(rng, M, K)
+    bits = lambda v: f32_to_bf16(np.array([v], dtype=np.float32))[0]
+    x[0, 7], x[1, K - 9], x[2, 11] = bits(np.inf), bits(-np.inf), bits(np.nan)
+    x[3, 5], x[3, K - 1] = bits(np.inf), bits(-np.inf)
+    x[4, 3], x[4, K // 2] = bits(-3e38), bits(1e38)
+    return x
+
+
+def _check_nonfinite(got16, x, w, s, b, bits, group, what):
+    """Outputs against the dequantized product in fp64: the same infinities and NaN, and
+    finite ones to the format's rounding (2 ** -7 of the row's largest)."""
+    from oracle import bf16_to_f32
+    from synth import deq_numpy
+
+    wd = deq_numpy(w, s, b, bits, group, fused=True).astype(np.float64)
+    with np.errstate(all="ignore"):
+        ref = bf16_to_f32(x).astype(np.float64) @ wd.T
+    got = bf16_to_f32(got16).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(ref)), what
+    assert np.array_equal(np.where(np.isinf(got), got, 0), np.where(np.isinf(ref), ref, 0)), what
+    ok = np.isfinite(ref)
+    for m in range(ref.shape[0]):
+        if ok[m].any():
+            top = np.abs(ref[m][ok[m]]).max()
+            assert np.abs(got[m] - ref[m])[ok[m]].max() <= 2 ** -7 * top, (what, m)
+
+
+@pytest.mark.parametrize("bits,M", [(4, 5), (4, 13), (4, 16), (8, 9), (8, 16)])
+@pytest.mark.parametrize("group", [32, 128])
+@pytest.mark.parametrize("N,K", [
+    (512, 512),     # K parts of two steps
+    (72, 1280),     # a ragged last tile, five steps
+    (8200, 1024),   # 32-row W tiles (4 bits), a ragged last one
+    (256, 8192),    # the pipelined walk
+])
+def test_quantized_matmul_nonfinite_rows(gpu, oracle, bits, group, M, N, K):
+    """Rows of x with infinities, NaN and values near the largest, in groups of 32 and 128
+    at one x tile: answered as by the dequantized weights, other rows untouched."""
+    from fastmlx_amd import ops
+
+    rng = np.random.default_rng(bits * 100 + group + M + N)
+    w, s, b = make_quant(rng, (N,), K, bits, group)
+    x = _nonfinite_x(rng, M, K)
+    announce(f"non-finite rows bits={bits} group={group} M={M} N={N} K={K}")
+    y = ops.quantized_matmul(to_dev(x, gpu), to_dev(w, gpu), to_dev(s, gpu), to_dev(b, gpu), True,
+                             group, bits)
+    torch.cuda.synchronize()
+    _check_nonfinite(to_np(y), x, w, s, b, bits, group, f"{bits} {group} {M} {N} {K}")
