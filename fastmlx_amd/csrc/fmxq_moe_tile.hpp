@@ -2,7 +2,9 @@
 // 64 slots of one expert by 4 x 32 columns of two matrices (gate and up), or 4 x 64
 // columns of one (down).  Same products, segment table, roundings and error handling
 // as the segment walk (fmxq_moe_walk.hpp), in exact affine arithmetic for every run
-// (the walk dequantizes pieces of 17 and more slots to bf16).
+// (the walk dequantizes pieces of 17 and more slots to bf16).  Outputs that come out
+// infinite or NaN so (an infinity in x, sums past the fp32 range) are taken again with
+// the dequantized weights.
 //
 // What bounds it: with few slots per expert the weight stream, with many the MFMA and
 // VALU work.  The walk's blocks (64 columns, 16 or 32 slots) are bound by the vector
@@ -385,33 +387,75 @@ __device__ __forceinline__ void tile_walk(const TileWave<BITS, GS>& tw, uint8_t*
   if (k < tw.steps) step(std::integral_constant<int, 0>{}, k);
 }
 
-template <int RT, int NMAT>
-__device__ __forceinline__ void tile_store(const MoeArgs& a, int64_t n0, int wave, int len, bool bad_e,
-                                           const uint32_t* rows, const f32x16 (&acc)[2][RT]) {
+template <int RT, int NMAT, int BITS, int GS>
+__device__ __forceinline__ void tile_store(const MoeArgs& a, int64_t start, int64_t eo, bool sh, int64_t n0,
+                                           int wave, int len, bool bad_e, const uint32_t* rows,
+                                           const f32x16 (&acc)[2][RT]) {
   const int lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5;
+  constexpr int NC = NMAT == 2 ? 1 : 2;  // stored columns per lane
+  auto column = [&](int c) { return n0 + 32 * kTileWaves * c + 32 * wave + r32; };
+  auto silu_mul = [&](float v0, float v1) {
+    const float g = tile_r16(v0), u = tile_r16(v1);
+    const float sg = tile_r16(1.f / (1.f + __expf(-g)));
+    return (uint16_t)f32_to_bf16_rne(tile_r16(tile_r16(g * sg) * u));
+  };
   // C layout: register r of lane l is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
+  auto row_of = [&](int i, int r) { return 32 * i + 8 * (r / 4) + 4 * h + (r % 4); };
+  // Infinite and NaN outputs, bit 16 i + r: one FMA per sum (0 times it, NaN then) tells
+  // a lane without any from the others.
+  uint32_t odd[NC] = {};
+  float zero = 0.f;
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) zero = __builtin_fmaf(acc[c][i][r], 0.f, zero);
+  if (__builtin_expect(zero != 0.f, 0)) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int m = row_of(i, r);
+          if (m < len && !bad_e && !(rows[m] >> 31) && column(c % NC) < a.N && !__builtin_isfinite(acc[c][i][r]))
+            odd[c % NC] |= 1u << (16 * i + r);
+        }
+  }
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const int m = 32 * i + 8 * (r / 4) + 4 * h + (r % 4);
+      const int m = row_of(i, r);
       if (m >= len) continue;
       const uint32_t row = rows[m];
       const bool bad = bad_e || (row >> 31);
       uint16_t* yr = a.y + (int64_t)(row & 0x7fffffffu) * a.N;
-      if constexpr (NMAT == 2) {
-        const int64_t n = n0 + 32 * wave + r32;
-        if (n >= a.N) continue;
-        const float g = tile_r16(acc[0][i][r]), u = tile_r16(acc[1][i][r]);
-        const float sg = tile_r16(1.f / (1.f + __expf(-g)));
-        yr[n] = bad ? 0 : (uint16_t)f32_to_bf16_rne(tile_r16(tile_r16(g * sg) * u));
-      } else {
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const int64_t n = n0 + 32 * kTileWaves * c + 32 * wave + r32;
-          if (n < a.N) yr[n] = bad ? 0 : (uint16_t)f32_to_bf16_rne(acc[c][i][r]);
-        }
+      for (int c = 0; c < NC; ++c) {
+        const int64_t n = column(c);
+        if (n >= a.N) continue;
+        const uint16_t v = NMAT == 2 ? silu_mul(acc[0][i][r], acc[1][i][r]) : (uint16_t)f32_to_bf16_rne(acc[c][i][r]);
+        yr[n] = bad ? 0 : v;
       }
+    }
+  // The walk's dequantized answers for rows whose sums are not finite (deq_row_dot).
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+    while (odd[c]) {
+      const int i = __builtin_ctz(odd[c]), r = i & 15;
+      odd[c] &= odd[c] - 1;
+      const int m = row_of(i >> 4, r);
+      const int64_t slot = start + m, n = eo + column(c);
+      const uint16_t* x = a.x + (a.lhs ? (int64_t)a.lhs[slot] : slot / a.lhs_div) * a.K;
+      float v[2] = {0.f, 0.f};
+#pragma unroll
+      for (int p = 0; p < NMAT; ++p)
+        v[p] = deq_row_dot<BITS, GS>(x, (sh ? a.sh_w[p] : a.w[p]) + n * (a.K * BITS / 32),
+                                     (sh ? a.sh_s[p] : a.s[p]) + n * (a.K / GS),
+                                     (sh ? a.sh_b[p] : a.b[p]) + n * (a.K / GS), 0, a.K);
+      a.y[(int64_t)rows[m] * a.N + column(c)] = NMAT == 2 ? silu_mul(v[0], v[1]) : (uint16_t)f32_to_bf16_rne(v[0]);
     }
 }
 
@@ -468,9 +512,10 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
   if (sg >= (int64_t)*a.nseg) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t start = a.seg[2 * sg];
-  const int len = (int)a.seg[2 * sg + 1];
-  const uint32_t e = a.rhs[start];
+  // One value per block: in scalar registers, which the walk has to spare.
+  const int64_t start = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.seg[2 * sg]);
+  const int len = __builtin_amdgcn_readfirstlane((int)a.seg[2 * sg + 1]);
+  const uint32_t e = (uint32_t)__builtin_amdgcn_readfirstlane((int)a.rhs[start]);
   const bool sh = a.sh_seg && (int64_t)e == a.E;
   const bool bad_e = (int64_t)e >= a.E && !sh;
   const int64_t n0 = (int64_t)blockIdx.x * (32 * kTileWaves * (NMAT == 2 ? 1 : 2));
@@ -533,11 +578,11 @@ __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu
   if (len <= 32) {
     f32x16 acc[2][1] = {};
     if (!bad_e) tile_walk<1, BITS, GS>(tw, xs0, xs1, stage[wave], sums0, sums1, wave, acc);
-    tile_store<1, NMAT>(a, n0, wave, len, bad_e, rows, acc);
+    tile_store<1, NMAT, BITS, GS>(a, start, eo, sh, n0, wave, len, bad_e, rows, acc);
   } else {
     f32x16 acc[2][2] = {};
     if (!bad_e) tile_walk<2, BITS, GS>(tw, xs0, xs1, stage[wave], sums0, sums1, wave, acc);
-    tile_store<2, NMAT>(a, n0, wave, len, bad_e, rows, acc);
+    tile_store<2, NMAT, BITS, GS>(a, start, eo, sh, n0, wave, len, bad_e, rows, acc);
   }
 }
 

@@ -1102,3 +1102,61 @@ def test_moe_layer_graph_replay(gpu, oracle):
         with torch.cuda.stream(side):  # eager work of another size between replays
             ops.moe_layer(xo[:2], io[:2], *dstack, wo[:2], dshared)
         torch.cuda.synchronize()
+
+
+# --- rows of x that are not finite, on the tiles ---
+
+@pytest.mark.parametrize("bits,group", [(4, 32), (4, 64), (4, 128), (8, 32), (8, 64), (8, 128)])
+def test_tiles_nonfinite_rows(gpu, oracle, bits, group):
+    """gather_qmm on the tiles (runs of 2100 and of 40 slots) with rows of x holding
+    infinities, NaN and values near the largest: answered as by the dequantized weights,
+    the other rows untouched."""
+    from fastmlx_amd import ops
+    from test_gpu_dense import _check_nonfinite, _nonfinite_x
+
+    rng = np.random.default_rng(bits + group)
+    E, N, K, xb = 4, 288, 512, 64
+    w, s, b = make_quant(rng, (E, N), K, bits, group)
+    x = _nonfinite_x(rng, xb, K)
+    rhs = np.concatenate([np.full(n, e, dtype=np.uint32) for e, n in enumerate((2100, 2100, 40, 31))])
+    lhs = np.arange(rhs.size, dtype=np.uint32) % xb
+    order = rng.permutation(rhs.size)
+    rhs, lhs = np.ascontiguousarray(rhs[order]), np.ascontiguousarray(lhs[order])
+    announce(f"tiles, non-finite rows, bits={bits} group={group}")
+    y = ops.gather_qmm(to_dev(x.reshape(xb, 1, K), gpu), to_dev(w, gpu), to_dev(s, gpu), to_dev(b, gpu),
+                       to_dev(rhs, gpu), to_dev(lhs, gpu), 1, True, group, bits, False)
+    torch.cuda.synchronize()
+    got = to_np(y).reshape(rhs.size, N)
+    for e in range(E):
+        at = np.nonzero(rhs == e)[0]
+        _check_nonfinite(got[at], x[lhs[at]], w[e], s[e], b[e], bits, group, f"expert {e}")
+
+
+@pytest.mark.parametrize("bits,group", [(4, 64), (4, 32), (8, 128)])
+def test_tiles_switch_glu_nonfinite_rows(gpu, oracle, bits, group):
+    """SwitchGLU on the tiles with every weight positive: an infinity in x makes gate, up,
+    their product and every output of that row +inf, a negative one NaN (silu(-inf) is
+    0 * -inf); values near the largest overflow to +inf; other rows equal the same call on
+    finite x bit for bit."""
+    from fastmlx_amd import ops
+
+    rng = np.random.default_rng(5)
+    E, T, k, D, I = 3, 2100, 2, 256, 512
+    stacks = []
+    for lead, K in (((E, I), D), ((E, I), D), ((E, D), I)):
+        w, s, _ = make_quant(rng, lead, K, bits, group)
+        stacks.append(tuple(to_dev(t, gpu) for t in (w, s, s)))  # (q + 1) s
+    x = torch.from_numpy(rng.standard_normal((T, D)).astype(np.float32)).bfloat16().to(gpu)
+    inds = to_dev(topk_uniform(rng, T, E, k).astype(np.uint32), gpu)
+    announce(f"switch_glu tiles, non-finite rows, bits={bits} group={group}")
+    plain = ops.switch_glu(x, inds, *stacks, group, bits)
+    odd = x.clone()
+    odd[3, 7], odd[4, 9] = float("inf"), float("-inf")
+    odd[5] = 0
+    odd[5, 100] = 3e38
+    got = ops.switch_glu(odd, inds, *stacks, group, bits)
+    torch.cuda.synchronize()
+    assert torch.isposinf(got[3]).all() and torch.isnan(got[4]).all() and torch.isposinf(got[5]).all()
+    rest = torch.ones(T, dtype=torch.bool)
+    rest[3:6] = False
+    assert torch.equal(got[rest], plain[rest])
