@@ -69,18 +69,23 @@ void retire(void* p) {
   g_retired.push_back(p);
 }
 
-int split_workspace(hipStream_t s, const fmxq::QmmPlan& plan, float** ws, uint32_t** cnt) {
+// Growth refused because the stream is being captured also sets *captured, for callers
+// that have another way to serve the call (hipMalloc failing does not).
+int split_workspace(hipStream_t s, const fmxq::QmmPlan& plan, float** ws, uint32_t** cnt,
+                    bool* captured = nullptr) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return fail(FMXQ_ERR_DEVICE, "hipGetDevice failed");
   std::lock_guard<std::mutex> lk(g_ws_mu);
   SplitWs& w = g_ws[{dev, s}];
   if (w.ws_floats < plan.ws_floats || w.n_counters < plan.tile_counters) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+      if (captured) *captured = true;
       return fail(FMXQ_ERR_INVALID_ARGUMENT,
                   "quantized_matmul: split-K workspace must grow to %lld floats during graph "
                   "capture; run the same shape once outside capture first",
                   (long long)plan.ws_floats);
+    }
     if (int rc = hip_status(hipStreamSynchronize(s), "split-K workspace: synchronize")) return rc;
     const int64_t nf = std::max(plan.ws_floats, w.ws_floats);
     const int64_t nc = std::max(plan.tile_counters, w.n_counters);
@@ -107,18 +112,20 @@ int split_workspace(hipStream_t s, const fmxq::QmmPlan& plan, float** ws, uint32
   return FMXQ_OK;
 }
 
-int prefill_workspace(hipStream_t s, int64_t floats, float** out) {
+int prefill_workspace(hipStream_t s, int64_t floats, float** out, bool* captured = nullptr) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return fail(FMXQ_ERR_DEVICE, "hipGetDevice failed");
   std::lock_guard<std::mutex> lk(g_ws_mu);
   SplitWs& w = g_ws[{dev, s}];
   if (w.pf_floats < floats) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+      if (captured) *captured = true;
       return fail(FMXQ_ERR_INVALID_ARGUMENT,
                   "quantized_matmul: prefill workspace must grow to %lld floats during graph "
                   "capture; run the same shape once outside capture first",
                   (long long)floats);
+    }
     if (int rc = hip_status(hipStreamSynchronize(s), "prefill workspace: synchronize")) return rc;
     float* p = nullptr;
     if (int rc = hip_status(hipMalloc(&p, floats * sizeof(float)), "prefill workspace: hipMalloc"))
@@ -297,6 +304,10 @@ int qmm_common(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
     return fail(FMXQ_ERR_INVALID_ARGUMENT, "%s: x and w must be 16-byte aligned", op);
   fmxq::QmmArgs a{x, w, scales, biases, bias, y, M, N, K, K, N, group_size, bits};
   hipStream_t s = static_cast<hipStream_t>(stream);
+  // Groups of 32 and 128 have other kernels for every size, which need no workspace or a
+  // smaller one: where the first choice would have to grow its own while the stream is
+  // being captured, they serve the call.
+  const bool others = group_size != 64;
   // Prefill sizes: the wide GEMM (256 x 256 tiles, weights dequantized in
   // registers, stream-K over the tiles past the last whole wave of blocks).
   if (fmxq::qmm_use_wide(M, N, K) && fmxq::qmm_wide_supported(a)) {
@@ -304,14 +315,18 @@ int qmm_common(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
     if (int rc = device_cus(&cus)) return rc;
     const fmxq::WidePlan wp = fmxq::qmm_wide_plan(M, N, K, cus);
     uint32_t* flag = nullptr;
+    bool captured = false;
+    int rc = FMXQ_OK;
     if (wp.sk_len > 0) {
-      if (int rc = prefill_workspace(s, wp.ws_floats, &a.ws)) return rc;
       float* unused = nullptr;
-      if (int rc = split_workspace(s, fmxq::QmmPlan{2, 0, wp.tiles}, &unused, &a.tile_count))
-        return rc;
-      if (int rc = device_flag(s, &flag)) return rc;
+      rc = prefill_workspace(s, wp.ws_floats, &a.ws, &captured);
+      if (!rc) rc = split_workspace(s, fmxq::QmmPlan{2, 0, wp.tiles}, &unused, &a.tile_count, &captured);
+      if (!rc) rc = device_flag(s, &flag);
     }
-    return hip_status(fmxq::launch_qmm_wide(a, wp, flag, s), op);
+    if (!rc) return hip_status(fmxq::launch_qmm_wide(a, wp, flag, s), op);
+    if (!captured || !others) return rc;
+    a.ws = nullptr;
+    a.tile_count = nullptr;
   }
   // qmvw, x shared through LDS and K split over blocks.  int4 group 64 at
   // 9 <= M <= 64, at M <= 16 only for wide outputs or long rows, where it beats
@@ -332,11 +347,14 @@ int qmm_common(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
     int cus = 0;
     if (int rc = device_cus(&cus)) return rc;
     const fmxq::QmvwPlan qp = fmxq::qmvw_plan(a, cus);
+    bool captured = false;
+    int rc = FMXQ_OK;
     if (qp.parts > 1) {
-      if (int rc = prefill_workspace(s, qp.ws_floats, &a.ws)) return rc;
-      a.splits = qp.parts;
+      rc = prefill_workspace(s, qp.ws_floats, &a.ws, &captured);
+      if (!rc) a.splits = qp.parts;
     }
-    return hip_status(fmxq::launch_qmvw(a, qp, s), op);
+    if (!rc) return hip_status(fmxq::launch_qmvw(a, qp, s), op);
+    if (!captured || !others) return rc;
   }
   // M <= 2: dot2 GEMV.  M = 3, 4: qmvs on outputs of 4096 rows or more (C1 stack,
   // 224 products, whose 1024-row k and v stay on the dot2 GEMV: M = 3 2.11 ->
