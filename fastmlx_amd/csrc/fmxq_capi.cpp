@@ -167,17 +167,21 @@ std::map<std::tuple<int, hipStream_t, int>, std::pair<void*, size_t>> g_arena;
 // Words of a zero-id buffer (fmxq_moe_layer, arena slot 3) already filled.
 std::map<const void*, int64_t> g_zero_filled;
 
-int stream_arena(hipStream_t s, size_t bytes, void** out, const char* op, int slot = 0) {
+// *captured: as in split_workspace.
+int stream_arena(hipStream_t s, size_t bytes, void** out, const char* op, int slot = 0,
+                 bool* captured = nullptr) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return fail(FMXQ_ERR_DEVICE, "hipGetDevice failed");
   std::lock_guard<std::mutex> lk(g_arena_mu);
   auto& a = g_arena[{dev, s, slot}];
   if (a.second < bytes) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone)
+    if (hipStreamIsCapturing(s, &cap) == hipSuccess && cap != hipStreamCaptureStatusNone) {
+      if (captured) *captured = true;
       return fail(FMXQ_ERR_INVALID_ARGUMENT,
                   "%s: scratch must grow to %zu bytes during graph capture; run the same shape "
                   "once outside capture first", op, bytes);
+    }
     void* p = nullptr;
     if (int rc = hip_status(hipMalloc(&p, bytes), "switch_glu scratch: hipMalloc")) return rc;
     retire(a.first);
@@ -194,8 +198,8 @@ int stream_arena(hipStream_t s, size_t bytes, void** out, const char* op, int sl
 struct ScratchSource {
   void* fixed = nullptr;
   size_t fixed_bytes = 0;
-  int get(hipStream_t s, size_t bytes, void** out, const char* op) const {
-    if (!fixed) return stream_arena(s, bytes, out, op);
+  int get(hipStream_t s, size_t bytes, void** out, const char* op, bool* captured = nullptr) const {
+    if (!fixed) return stream_arena(s, bytes, out, op, 0, captured);
     if (bytes > fixed_bytes)
       return fail(FMXQ_ERR_SHAPE,
                   "%s: this call needs %zu bytes of scratch, more than the %zu bytes the "
@@ -227,7 +231,8 @@ struct MoeScratch {
 };
 int moe_scratch(hipStream_t s, int64_t S, int64_t h_cols, int64_t max_seg, MoeScratch* m,
                 const char* op, int64_t max_tiles = 0, int64_t gu_cols = 0,
-                const ScratchSource& src = ScratchSource(), int64_t prep = 0) {
+                const ScratchSource& src = ScratchSource(), int64_t prep = 0,
+                bool* captured = nullptr) {
   const size_t ib = align_up((size_t)S * sizeof(uint32_t));
   const size_t sb = align_up((size_t)max_seg * 2 * sizeof(uint32_t));
   const size_t hb = align_up((size_t)S * h_cols * sizeof(uint16_t));
@@ -235,7 +240,8 @@ int moe_scratch(hipStream_t s, int64_t S, int64_t h_cols, int64_t max_seg, MoeSc
   const size_t gb = align_up((size_t)S * gu_cols * sizeof(uint16_t));
   void* arena = nullptr;
   const size_t pb = align_up((size_t)prep);
-  if (int rc = src.get(s, 3 * ib + sb + 256 + hb + tb + 256 + 2 * gb + pb, &arena, op)) return rc;
+  if (int rc = src.get(s, 3 * ib + sb + 256 + hb + tb + 256 + 2 * gb + pb, &arena, op, captured))
+    return rc;
   char* p = static_cast<char*>(arena);
   m->order = reinterpret_cast<uint32_t*>(p);
   m->rhs = reinterpret_cast<uint32_t*>(p + ib);
@@ -544,18 +550,16 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
                       group_size, bits, lhs_div};
       return hip_status(fmxq::launch_moe_qmvs(a, 1, 16, batch, s), op);
     }
-    const int window = fmxq::moe_window(batch, E, N, K, N, K, x_batch, bits, group_size);
-    const int64_t max_seg = fmxq::moe_max_segments(batch, E, window);
-    if (max_seg <= kMaxSegmentsGrid) {
+    // Sorted, in segments of `window` slots (the caller has checked their count).
+    auto sorted = [&](int window, int64_t max_seg, bool* captured) -> int {
       MoeScratch m;
-      const int64_t max_tiles = window != fmxq::kMoeTileRows &&
-                                        fmxq::qmm_grouped_supported(N, K, x_batch, bits, group_size)
+      const bool tile = window == fmxq::kMoeTileRows;
+      const int64_t max_tiles = !tile && fmxq::qmm_grouped_supported(N, K, x_batch, bits, group_size)
                                     ? grouped_max_tiles(batch, E)
                                     : 0;
-      const int64_t prep = window == fmxq::kMoeTileRows
-                               ? fmxq::moe_tile_prep_bytes(x_batch * K, bits, group_size)
-                               : 0;
-      if (int rc = moe_scratch(s, batch, 0, max_seg, &m, op, max_tiles, 0, ScratchSource(), prep))
+      const int64_t prep = tile ? fmxq::moe_tile_prep_bytes(x_batch * K, bits, group_size) : 0;
+      if (int rc = moe_scratch(s, batch, 0, max_seg, &m, op, max_tiles, 0, ScratchSource(), prep,
+                               captured))
         return rc;
       if (int rc = hip_status(fmxq::launch_sort_slots(rhs_indices, batch, lhs_div, E, m.order,
                                                       m.rhs, m.lhs, s, lhs_indices, m.seg,
@@ -572,6 +576,18 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
       const fmxq::QmmArgs gq = grouped_args(x, w, scales, biases, y, N, K, bits, group_size, m,
                                             m.lhs, m.order, x_batch, flag);
       return hip_status(fmxq::launch_qmm_grouped(gq, max_tiles, s), op);
+    };
+    // Where the stream is being captured and its scratch would have to grow, the next
+    // window that needs less, then (formats other than 4 bits in groups of 64, whose
+    // general kernels need none) the kernels below.
+    const int first = fmxq::moe_window(batch, E, N, K, N, K, x_batch, bits, group_size);
+    const int walk = fmxq::moe_walk_window(batch, E);
+    for (int window : {first, walk}) {
+      const int64_t max_seg = fmxq::moe_max_segments(batch, E, window);
+      if (max_seg > kMaxSegmentsGrid) continue;
+      bool captured = false;
+      const int rc = sorted(window, max_seg, &captured);
+      if (!captured || (window == walk && bits == 4 && group_size == 64)) return rc;
     }
   }
   fmxq::GatherArgs a{x,      w,     scales,  biases, lhs_indices, rhs_indices, y,
@@ -649,19 +665,17 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
   if (int rc = device_flag(static_cast<hipStream_t>(stream), &flag)) return rc;
   // The tiles keep a prepared copy of x, then of h; where the fixed scratch of the
   // allocation-free call does not hold it, the walk takes the batch.
-  int window = fmxq::moe_window(S, E, I, D, D, I, std::max(S, T), bits, group_size);
-  int64_t prep = 0;
-  if (window == fmxq::kMoeTileRows) {
-    prep = fmxq::moe_tile_prep_bytes(std::max(T * D, S * I), bits, group_size);
-    const int64_t rest = 2 * S * I + 12 * S + 16 * (S + E) + 4096;
-    if (src.fixed && prep + rest > (int64_t)src.fixed_bytes) {
-      window = fmxq::moe_walk_window(S, E);
-      prep = 0;
-    }
-  }
-  const int64_t max_seg = fmxq::moe_max_segments(S, E, window);
-  if (E <= kSortMaxExperts && max_seg <= kMaxSegmentsGrid &&
-      fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
+  int first = fmxq::moe_window(S, E, I, D, D, I, std::max(S, T), bits, group_size);
+  const int walk = fmxq::moe_walk_window(S, E);
+  const int64_t prep_bytes = fmxq::moe_tile_prep_bytes(std::max(T * D, S * I), bits, group_size);
+  if (first == fmxq::kMoeTileRows && src.fixed &&
+      prep_bytes + 2 * S * I + 12 * S + 16 * (S + E) + 4096 > (int64_t)src.fixed_bytes)
+    first = walk;
+  // Where the stream is being captured and its scratch would have to grow, the walk, which
+  // needs less than the tiles, then (formats other than 4 bits in groups of 64) the
+  // general kernels below.
+  const bool others = bits != 4 || group_size != 64;
+  if (E <= kSortMaxExperts && fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
       fmxq::moe_qmvs_supported(D, I, S + T, bits, group_size) && aligned16(s_gate) &&
       aligned16(b_gate) && aligned16(s_up) && aligned16(b_up) && aligned16(s_down) &&
       aligned16(b_down)) {
@@ -669,9 +683,9 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
     // slot being its own product row), then gate and up fused with silu * up into
     // h in sorted order, then down written to each slot's own output row.  A few
     // slots skip the sort: each is its own segment, h stays in slot order.
-    MoeScratch m;
-    if (S <= fmxq::kMoeUnsortedMaxSlots) {
-      if (int rc = moe_scratch(s, S, I, 1, &m, op, 0, 0, src)) return rc;
+    auto unsorted = [&](bool* captured) -> int {
+      MoeScratch m;
+      if (int rc = moe_scratch(s, S, I, 1, &m, op, 0, 0, src, 0, captured)) return rc;
       fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
                        nullptr, m.h, nullptr, S, I, D, E, T, flag, group_size, bits, topk};
       if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, 16, S, s), "switch_glu: gate/up"))
@@ -679,52 +693,70 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
       fmxq::MoeArgs dn{m.h, nullptr, {w_down, nullptr}, {s_down, nullptr}, {b_down, nullptr},
                        inds, nullptr, nullptr, out, nullptr, S, D, I, E, S, flag, group_size, bits, 1};
       return hip_status(fmxq::launch_moe_qmvs(dn, 1, 16, S, s), "switch_glu: down");
+    };
+    auto sorted = [&](int window, int64_t max_seg, bool* captured) -> int {
+      MoeScratch m;
+      const bool tile = window == fmxq::kMoeTileRows;
+      // Long expert runs (>= kGroupedMinRun slots) go to the grouped GEMM: gate and
+      // up into g and u, silu * up into their h rows, then down.
+      const int64_t max_tiles =
+          !tile && fmxq::qmm_grouped_supported(I, D, T, bits, group_size) &&
+                  fmxq::qmm_grouped_supported(D, I, S, bits, group_size)
+              ? grouped_max_tiles(S, E)
+              : 0;
+      if (int rc = moe_scratch(s, S, I, max_seg, &m, op, max_tiles, max_tiles ? I : 0, src,
+                               tile ? prep_bytes : 0, captured))
+        return rc;
+      if (int rc = hip_status(fmxq::launch_sort_slots(inds, S, topk, E, m.order, m.rhs, m.lhs, s,
+                                                      nullptr, m.seg, m.nseg, window, m.tiles,
+                                                      m.ntile, (int)kGroupedMinRun,
+                                                      fmxq::kGroupedTileRows),
+                              "switch_glu: sort"))
+        return rc;
+      fmxq::MoeArgs gu{x, m.lhs, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, m.rhs, m.seg,
+                       m.nseg, m.h, nullptr, S, I, D, E, T, flag, group_size, bits};
+      gu.xprep = m.xprep;
+      if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, window, max_seg, s),
+                              "switch_glu: gate/up"))
+        return rc;
+      if (max_tiles) {
+        const fmxq::QmmArgs gg = grouped_args(x, w_gate, s_gate, b_gate, m.g, I, D, bits,
+                                              group_size, m, m.lhs, nullptr, T, flag);
+        if (int rc = hip_status(fmxq::launch_qmm_grouped(gg, max_tiles, s), "switch_glu: gate"))
+          return rc;
+        const fmxq::QmmArgs gup = grouped_args(x, w_up, s_up, b_up, m.u, I, D, bits, group_size,
+                                               m, m.lhs, nullptr, T, flag);
+        if (int rc = hip_status(fmxq::launch_qmm_grouped(gup, max_tiles, s), "switch_glu: up"))
+          return rc;
+        if (int rc = hip_status(fmxq::launch_silu_mul_tiles(m.g, m.u, m.h, m.tiles, m.ntile,
+                                                            max_tiles, fmxq::kGroupedTileRows, I,
+                                                            s),
+                                "switch_glu: silu"))
+          return rc;
+      }
+      fmxq::MoeArgs dn{m.h, nullptr, {w_down, nullptr}, {s_down, nullptr}, {b_down, nullptr},
+                       m.rhs, m.seg, m.nseg, out, m.order, S, D, I, E, S, flag, group_size, bits};
+      dn.xprep = m.xprep;
+      if (int rc = hip_status(fmxq::launch_moe_qmvs(dn, 1, window, max_seg, s), "switch_glu: down"))
+        return rc;
+      if (!max_tiles) return FMXQ_OK;
+      const fmxq::QmmArgs gd = grouped_args(m.h, w_down, s_down, b_down, out, D, I, bits,
+                                            group_size, m, nullptr, m.order, S, flag);
+      return hip_status(fmxq::launch_qmm_grouped(gd, max_tiles, s), "switch_glu: down");
+    };
+    if (S <= fmxq::kMoeUnsortedMaxSlots) {
+      bool captured = false;
+      const int rc = unsorted(&captured);
+      if (!captured || !others) return rc;
+    } else {
+      for (int window : {first, walk}) {
+        const int64_t max_seg = fmxq::moe_max_segments(S, E, window);
+        if (max_seg > kMaxSegmentsGrid) continue;
+        bool captured = false;
+        const int rc = sorted(window, max_seg, &captured);
+        if (!captured || (window == walk && !others)) return rc;
+      }
     }
-    // Long expert runs (>= kGroupedMinRun slots) go to the grouped GEMM: gate and
-    // up into g and u, silu * up into their h rows, then down.
-    const int64_t max_tiles =
-        window != fmxq::kMoeTileRows && fmxq::qmm_grouped_supported(I, D, T, bits, group_size) &&
-                fmxq::qmm_grouped_supported(D, I, S, bits, group_size)
-            ? grouped_max_tiles(S, E)
-            : 0;
-    if (int rc = moe_scratch(s, S, I, max_seg, &m, op, max_tiles, max_tiles ? I : 0, src, prep))
-      return rc;
-    if (int rc = hip_status(fmxq::launch_sort_slots(inds, S, topk, E, m.order, m.rhs, m.lhs, s,
-                                                    nullptr, m.seg, m.nseg, window, m.tiles,
-                                                    m.ntile, (int)kGroupedMinRun,
-                                                    fmxq::kGroupedTileRows),
-                            "switch_glu: sort"))
-      return rc;
-    fmxq::MoeArgs gu{x, m.lhs, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, m.rhs, m.seg,
-                     m.nseg, m.h, nullptr, S, I, D, E, T, flag, group_size, bits};
-    gu.xprep = m.xprep;
-    if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, window, max_seg, s),
-                            "switch_glu: gate/up"))
-      return rc;
-    if (max_tiles) {
-      const fmxq::QmmArgs gg = grouped_args(x, w_gate, s_gate, b_gate, m.g, I, D, bits,
-                                            group_size, m, m.lhs, nullptr, T, flag);
-      if (int rc = hip_status(fmxq::launch_qmm_grouped(gg, max_tiles, s), "switch_glu: gate"))
-        return rc;
-      const fmxq::QmmArgs gup = grouped_args(x, w_up, s_up, b_up, m.u, I, D, bits, group_size,
-                                             m, m.lhs, nullptr, T, flag);
-      if (int rc = hip_status(fmxq::launch_qmm_grouped(gup, max_tiles, s), "switch_glu: up"))
-        return rc;
-      if (int rc = hip_status(fmxq::launch_silu_mul_tiles(m.g, m.u, m.h, m.tiles, m.ntile,
-                                                          max_tiles, fmxq::kGroupedTileRows, I,
-                                                          s),
-                              "switch_glu: silu"))
-        return rc;
-    }
-    fmxq::MoeArgs dn{m.h, nullptr, {w_down, nullptr}, {s_down, nullptr}, {b_down, nullptr},
-                     m.rhs, m.seg, m.nseg, out, m.order, S, D, I, E, S, flag, group_size, bits};
-    dn.xprep = m.xprep;
-    if (int rc = hip_status(fmxq::launch_moe_qmvs(dn, 1, window, max_seg, s), "switch_glu: down"))
-      return rc;
-    if (!max_tiles) return FMXQ_OK;
-    const fmxq::QmmArgs gd = grouped_args(m.h, w_down, s_down, b_down, out, D, I, bits,
-                                          group_size, m, nullptr, m.order, S, flag);
-    return hip_status(fmxq::launch_qmm_grouped(gd, max_tiles, s), "switch_glu: down");
   }
   // The reference sorts once routing reaches 64 slots (switch_glu.go:119-124).
   const bool sort = S >= 64 && E <= kSortMaxExperts;
@@ -825,15 +857,19 @@ extern "C" int fmxq_switch_glu_combine(
     uint32_t* flag = nullptr;
     if (int rc = device_flag(static_cast<hipStream_t>(stream), &flag)) return rc;
     MoeScratch m;
-    if (int rc = moe_scratch(s, S, I, 1, &m, op)) return rc;
-    fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
-                     nullptr, m.h, nullptr, S, I, D, E, T, flag, group_size, bits, topk};
-    if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, 16, S, s), "switch_glu_combine: gate/up"))
-      return rc;
-    return hip_status(fmxq::launch_moe_down_combine(m.h, inds, w_down, s_down, b_down, weights,
-                                                    shared, shared_gate, out, T, topk, E, D, I,
-                                                    group_size, bits, flag, s),
-                      "switch_glu_combine: down/combine");
+    bool captured = false;
+    const int rc = moe_scratch(s, S, I, 1, &m, op, 0, 0, ScratchSource(), 0, &captured);
+    if (rc && !captured) return rc;
+    if (!rc) {
+      fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
+                       nullptr, m.h, nullptr, S, I, D, E, T, flag, group_size, bits, topk};
+      if (int e = hip_status(fmxq::launch_moe_qmvs(gu, 2, 16, S, s), "switch_glu_combine: gate/up"))
+        return e;
+      return hip_status(fmxq::launch_moe_down_combine(m.h, inds, w_down, s_down, b_down, weights,
+                                                      shared, shared_gate, out, T, topk, E, D, I,
+                                                      group_size, bits, flag, s),
+                        "switch_glu_combine: down/combine");
+    }
   }
   // Otherwise the two calls in sequence, the expert rows in the arena's slot 1.
   void* rows = nullptr;
@@ -888,22 +924,27 @@ extern "C" int fmxq_moe_layer(
     uint32_t* flag = nullptr;
     if (int rc = device_flag(s, &flag)) return rc;
     MoeScratch m;
-    if (int rc = moe_scratch(s, S + T, I, 1, &m, op)) return rc;
-    fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
-                     nullptr, m.h, nullptr, S, I, D, E, T, flag, group_size, bits, topk};
-    gu.sh_w[0] = sw_gate;
-    gu.sh_w[1] = sw_up;
-    gu.sh_s[0] = ss_gate;
-    gu.sh_s[1] = ss_up;
-    gu.sh_b[0] = sb_gate;
-    gu.sh_b[1] = sb_up;
-    gu.sh_T = T;
-    if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, 16, S, s), "moe_layer: gate/up"))
-      return rc;
-    return hip_status(fmxq::launch_moe_down_combine(m.h, inds, w_down, s_down, b_down, weights,
-                                                    nullptr, shared_gate, out, T, topk, E, D, I,
-                                                    group_size, bits, flag, s, sw_down, ss_down, sb_down),
-                      "moe_layer: down/combine");
+    bool captured = false;
+    const int rc = moe_scratch(s, S + T, I, 1, &m, op, 0, 0, ScratchSource(), 0, &captured);
+    if (rc && !captured) return rc;
+    if (!rc) {
+      fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
+                       nullptr, m.h, nullptr, S, I, D, E, T, flag, group_size, bits, topk};
+      gu.sh_w[0] = sw_gate;
+      gu.sh_w[1] = sw_up;
+      gu.sh_s[0] = ss_gate;
+      gu.sh_s[1] = ss_up;
+      gu.sh_b[0] = sb_gate;
+      gu.sh_b[1] = sb_up;
+      gu.sh_T = T;
+      if (int e = hip_status(fmxq::launch_moe_qmvs(gu, 2, 16, S, s), "moe_layer: gate/up"))
+        return e;
+      return hip_status(fmxq::launch_moe_down_combine(m.h, inds, w_down, s_down, b_down, weights,
+                                                      nullptr, shared_gate, out, T, topk, E, D, I,
+                                                      group_size, bits, flag, s, sw_down, ss_down,
+                                                      sb_down),
+                        "moe_layer: down/combine");
+    }
   }
   // Sorted batches below the grouped GEMM's floor: the shared expert joins the
   // sort as expert id E with one slot per token (after the S routed slots), so its
@@ -913,26 +954,9 @@ extern "C" int fmxq_moe_layer(
     const int64_t Sa = S + T;
     const int window = fmxq::moe_window(Sa, E + 1, I, D, D, I, Sa, bits, group_size);
     const int64_t max_seg = fmxq::moe_max_segments(Sa, E + 1, window);
-    if (!fmxq::moe_combine_unsorted(S, E) &&
-        (window == fmxq::kMoeTileRows || grouped_max_tiles(S, E) == 0) &&
-        E + 1 <= kSortMaxExperts && max_seg <= kMaxSegmentsGrid &&
-        fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
-        fmxq::moe_qmvs_supported(D, I, S + T, bits, group_size) && aligned16(s_gate) &&
-        aligned16(b_gate) && aligned16(s_up) && aligned16(b_up) && aligned16(s_down) &&
-        aligned16(b_down) && aligned16(ss_gate) && aligned16(sb_gate) && aligned16(ss_up) &&
-        aligned16(sb_up) && aligned16(ss_down) && aligned16(sb_down)) {
+    auto layer = [&](const MoeScratch& m, uint16_t* y) -> int {
       uint32_t* flag = nullptr;
       if (int rc = device_flag(s, &flag)) return rc;
-      MoeScratch m;
-      const int64_t prep =
-          window == fmxq::kMoeTileRows
-              ? fmxq::moe_tile_prep_bytes(std::max(T * D, Sa * I), bits, group_size)
-              : 0;
-      if (int rc = moe_scratch(s, Sa, I, max_seg, &m, op, 0, 0, ScratchSource(), prep)) return rc;
-      void* rows = nullptr;
-      if (int rc = stream_arena(s, align_up((size_t)Sa * D * sizeof(uint16_t)), &rows, op, 1))
-        return rc;
-      uint16_t* y = static_cast<uint16_t*>(rows);
       if (int rc = hip_status(fmxq::launch_sort_slots(inds, S, topk, E, m.order, m.rhs, m.lhs, s,
                                                       nullptr, m.seg, m.nseg, window, nullptr,
                                                       nullptr, 0, 0, T),
@@ -963,6 +987,27 @@ extern "C" int fmxq_moe_layer(
       return hip_status(fmxq::launch_moe_combine(y, weights, y + S * D, shared_gate, out, T, topk,
                                                  D, s),
                         "moe_layer: combine");
+    };
+    if (!fmxq::moe_combine_unsorted(S, E) &&
+        (window == fmxq::kMoeTileRows || grouped_max_tiles(S, E) == 0) &&
+        E + 1 <= kSortMaxExperts && max_seg <= kMaxSegmentsGrid &&
+        fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
+        fmxq::moe_qmvs_supported(D, I, S + T, bits, group_size) && aligned16(s_gate) &&
+        aligned16(b_gate) && aligned16(s_up) && aligned16(b_up) && aligned16(s_down) &&
+        aligned16(b_down) && aligned16(ss_gate) && aligned16(sb_gate) && aligned16(ss_up) &&
+        aligned16(sb_up) && aligned16(ss_down) && aligned16(sb_down)) {
+      MoeScratch m;
+      const int64_t prep =
+          window == fmxq::kMoeTileRows
+              ? fmxq::moe_tile_prep_bytes(std::max(T * D, Sa * I), bits, group_size)
+              : 0;
+      void* rows = nullptr;
+      bool captured = false;
+      int rc = moe_scratch(s, Sa, I, max_seg, &m, op, 0, 0, ScratchSource(), prep, &captured);
+      if (!rc)
+        rc = stream_arena(s, align_up((size_t)Sa * D * sizeof(uint16_t)), &rows, op, 1, &captured);
+      if (rc && !captured) return rc;
+      if (!rc) return layer(m, static_cast<uint16_t*>(rows));
     }
   }
   // Otherwise the shared expert as a one-expert SwitchGLU over every token (its

@@ -86,6 +86,9 @@ int fmxq_dequantize_rows(const uint32_t* w, const uint16_t* scales, const uint16
 
 /* y [M, N] = x [M, K] . deq(W)^T, fp32 accumulation, bf16 output.
  * transpose must be true (the only value the reference passes, quant.go:98).
+ * Some shapes sum partial products in a per-stream workspace, grown on first use.
+ * While the stream is being captured into a graph it cannot grow: groups of 32
+ * and 128 then run on kernels that fit, groups of 64 are refused.
  * Replaces mlx_quantized_matmul (mlxgo/binding_cgo.go:636-643). */
 int fmxq_quantized_matmul(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
                           const uint16_t* biases, uint16_t* y, int64_t M, int64_t N,
@@ -142,7 +145,9 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
  * and scattered back to token order (the sorted branch, :135-150).  Each op's
  * result is rounded to bf16 as in the reference chain (gather_qmm, sigmoid,
  * mul, mul).  Intermediates live in a per-stream scratch area the library
- * grows on first use of a shape (not allowed during graph capture).
+ * grows on first use of a shape.  It cannot grow while the stream is being
+ * captured into a graph: a call there takes a path that fits what the stream
+ * holds, and is refused if there is none.
  * Out-of-range expert ids give zero rows and raise the fmxq_device_error flag. */
 int fmxq_switch_glu(const uint16_t* x, const uint32_t* inds, const uint32_t* w_gate,
                     const uint16_t* s_gate, const uint16_t* b_gate, const uint32_t* w_up,
