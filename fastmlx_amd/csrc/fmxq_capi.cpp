@@ -229,19 +229,26 @@ struct MoeScratch {
   uint16_t *g = nullptr, *u = nullptr;
   uint8_t* xprep = nullptr;  // with prep > 0: that many bytes for the tiles' x
 };
+struct MoeScratchBytes {
+  size_t ib, sb, hb, tb, gb, pb;
+  MoeScratchBytes(int64_t S, int64_t h_cols, int64_t max_seg, int64_t max_tiles, int64_t gu_cols,
+                  int64_t prep)
+      : ib(align_up((size_t)S * sizeof(uint32_t))),
+        sb(align_up((size_t)max_seg * 2 * sizeof(uint32_t))),
+        hb(align_up((size_t)S * h_cols * sizeof(uint16_t))),
+        tb(align_up((size_t)max_tiles * 2 * sizeof(uint32_t))),
+        gb(align_up((size_t)S * gu_cols * sizeof(uint16_t))),
+        pb(align_up((size_t)prep)) {}
+  size_t total() const { return 3 * ib + sb + 256 + hb + tb + 256 + 2 * gb + pb; }
+};
 int moe_scratch(hipStream_t s, int64_t S, int64_t h_cols, int64_t max_seg, MoeScratch* m,
                 const char* op, int64_t max_tiles = 0, int64_t gu_cols = 0,
                 const ScratchSource& src = ScratchSource(), int64_t prep = 0,
                 bool* captured = nullptr) {
-  const size_t ib = align_up((size_t)S * sizeof(uint32_t));
-  const size_t sb = align_up((size_t)max_seg * 2 * sizeof(uint32_t));
-  const size_t hb = align_up((size_t)S * h_cols * sizeof(uint16_t));
-  const size_t tb = align_up((size_t)max_tiles * 2 * sizeof(uint32_t));
-  const size_t gb = align_up((size_t)S * gu_cols * sizeof(uint16_t));
+  const MoeScratchBytes z(S, h_cols, max_seg, max_tiles, gu_cols, prep);
+  const size_t ib = z.ib, sb = z.sb, hb = z.hb, tb = z.tb, gb = z.gb;
   void* arena = nullptr;
-  const size_t pb = align_up((size_t)prep);
-  if (int rc = src.get(s, 3 * ib + sb + 256 + hb + tb + 256 + 2 * gb + pb, &arena, op, captured))
-    return rc;
+  if (int rc = src.get(s, z.total(), &arena, op, captured)) return rc;
   char* p = static_cast<char*>(arena);
   m->order = reinterpret_cast<uint32_t*>(p);
   m->rhs = reinterpret_cast<uint32_t*>(p + ib);
@@ -663,14 +670,12 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
   hipStream_t s = static_cast<hipStream_t>(stream);
   uint32_t* flag = nullptr;
   if (int rc = device_flag(static_cast<hipStream_t>(stream), &flag)) return rc;
-  // The tiles keep a prepared copy of x, then of h; where the fixed scratch of the
-  // allocation-free call does not hold it, the walk takes the batch.
-  int first = fmxq::moe_window(S, E, I, D, D, I, std::max(S, T), bits, group_size);
+  const int first = fmxq::moe_window(S, E, I, D, D, I, std::max(S, T), bits, group_size);
   const int walk = fmxq::moe_walk_window(S, E);
-  const int64_t prep_bytes = fmxq::moe_tile_prep_bytes(std::max(T * D, S * I), bits, group_size);
-  if (first == fmxq::kMoeTileRows && src.fixed &&
-      prep_bytes + 2 * S * I + 12 * S + 16 * (S + E) + 4096 > (int64_t)src.fixed_bytes)
-    first = walk;
+  // The tiles keep a prepared copy of x, then of h.
+  auto prep_bytes = [&](int64_t nt) {
+    return fmxq::moe_tile_prep_bytes(std::max(nt * D, nt * topk * I), bits, group_size);
+  };
   // Where the stream is being captured and its scratch would have to grow, the walk, which
   // needs less than the tiles, then (formats other than 4 bits in groups of 64) the
   // general kernels below.
@@ -694,8 +699,12 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
                        inds, nullptr, nullptr, out, nullptr, S, D, I, E, S, flag, group_size, bits, 1};
       return hip_status(fmxq::launch_moe_qmvs(dn, 1, 16, S, s), "switch_glu: down");
     };
-    auto sorted = [&](int window, int64_t max_seg, bool* captured) -> int {
+    // Tokens t0 .. t0 + nt, in segments of `window` slots.
+    auto sorted = [&](int window, int64_t t0, int64_t nt, bool* captured) -> int {
       MoeScratch m;
+      const int64_t T = nt, S = nt * topk, max_seg = fmxq::moe_max_segments(S, E, window);
+      const uint16_t* const xt = x + t0 * D;
+      uint16_t* const yt = out + t0 * topk * D;
       const bool tile = window == fmxq::kMoeTileRows;
       // Long expert runs (>= kGroupedMinRun slots) go to the grouped GEMM: gate and
       // up into g and u, silu * up into their h rows, then down.
@@ -705,26 +714,26 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
               ? grouped_max_tiles(S, E)
               : 0;
       if (int rc = moe_scratch(s, S, I, max_seg, &m, op, max_tiles, max_tiles ? I : 0, src,
-                               tile ? prep_bytes : 0, captured))
+                               tile ? prep_bytes(nt) : 0, captured))
         return rc;
-      if (int rc = hip_status(fmxq::launch_sort_slots(inds, S, topk, E, m.order, m.rhs, m.lhs, s,
+      if (int rc = hip_status(fmxq::launch_sort_slots(inds + t0 * topk, S, topk, E, m.order, m.rhs, m.lhs, s,
                                                       nullptr, m.seg, m.nseg, window, m.tiles,
                                                       m.ntile, (int)kGroupedMinRun,
                                                       fmxq::kGroupedTileRows),
                               "switch_glu: sort"))
         return rc;
-      fmxq::MoeArgs gu{x, m.lhs, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, m.rhs, m.seg,
+      fmxq::MoeArgs gu{xt, m.lhs, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, m.rhs, m.seg,
                        m.nseg, m.h, nullptr, S, I, D, E, T, flag, group_size, bits};
       gu.xprep = m.xprep;
       if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, window, max_seg, s),
                               "switch_glu: gate/up"))
         return rc;
       if (max_tiles) {
-        const fmxq::QmmArgs gg = grouped_args(x, w_gate, s_gate, b_gate, m.g, I, D, bits,
+        const fmxq::QmmArgs gg = grouped_args(xt, w_gate, s_gate, b_gate, m.g, I, D, bits,
                                               group_size, m, m.lhs, nullptr, T, flag);
         if (int rc = hip_status(fmxq::launch_qmm_grouped(gg, max_tiles, s), "switch_glu: gate"))
           return rc;
-        const fmxq::QmmArgs gup = grouped_args(x, w_up, s_up, b_up, m.u, I, D, bits, group_size,
+        const fmxq::QmmArgs gup = grouped_args(xt, w_up, s_up, b_up, m.u, I, D, bits, group_size,
                                                m, m.lhs, nullptr, T, flag);
         if (int rc = hip_status(fmxq::launch_qmm_grouped(gup, max_tiles, s), "switch_glu: up"))
           return rc;
@@ -735,12 +744,12 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
           return rc;
       }
       fmxq::MoeArgs dn{m.h, nullptr, {w_down, nullptr}, {s_down, nullptr}, {b_down, nullptr},
-                       m.rhs, m.seg, m.nseg, out, m.order, S, D, I, E, S, flag, group_size, bits};
+                       m.rhs, m.seg, m.nseg, yt, m.order, S, D, I, E, S, flag, group_size, bits};
       dn.xprep = m.xprep;
       if (int rc = hip_status(fmxq::launch_moe_qmvs(dn, 1, window, max_seg, s), "switch_glu: down"))
         return rc;
       if (!max_tiles) return FMXQ_OK;
-      const fmxq::QmmArgs gd = grouped_args(m.h, w_down, s_down, b_down, out, D, I, bits,
+      const fmxq::QmmArgs gd = grouped_args(m.h, w_down, s_down, b_down, yt, D, I, bits,
                                             group_size, m, nullptr, m.order, S, flag);
       return hip_status(fmxq::launch_qmm_grouped(gd, max_tiles, s), "switch_glu: down");
     };
@@ -749,11 +758,31 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
       const int rc = unsorted(&captured);
       if (!captured || !others) return rc;
     } else {
+      if (src.fixed && first == fmxq::kMoeTileRows) {
+        // The fixed scratch may not hold the prepared copies: then the tokens in as few
+        // equal parts as do, each on the tiles, so that the values are those of the
+        // allocating call (the walk, which dequantizes longer runs, would round
+        // otherwise).  The whole batch's h rows and slots have to fit all the same.
+        const int64_t walk_seg = fmxq::moe_max_segments(S, E, walk);
+        void* unused = nullptr;
+        if (int rc = src.get(s, MoeScratchBytes(S, I, walk_seg, 0, 0, 0).total(), &unused, op)) return rc;
+        int64_t parts = 1, nt = T;
+        auto bytes = [&](int64_t n) {
+          return MoeScratchBytes(n * topk, I, fmxq::moe_max_segments(n * topk, E, first), 0, 0,
+                                 prep_bytes(n)).total();
+        };
+        while (nt > 1 && bytes(nt) > src.fixed_bytes) nt = (T + parts) / (parts + 1), ++parts;
+        if (bytes(nt) <= src.fixed_bytes && fmxq::moe_max_segments(nt * topk, E, first) <= kMaxSegmentsGrid) {
+          for (int64_t t0 = 0; t0 < T; t0 += nt)
+            if (int rc = sorted(first, t0, std::min(nt, T - t0), nullptr)) return rc;
+          return FMXQ_OK;
+        }
+      }
       for (int window : {first, walk}) {
-        const int64_t max_seg = fmxq::moe_max_segments(S, E, window);
-        if (max_seg > kMaxSegmentsGrid) continue;
+        if (fmxq::moe_max_segments(S, E, window) > kMaxSegmentsGrid) continue;
+        if (src.fixed && window == fmxq::kMoeTileRows) continue;  // no part fits
         bool captured = false;
-        const int rc = sorted(window, max_seg, &captured);
+        const int rc = sorted(window, 0, T, &captured);
         if (!captured || (window == walk && !others)) return rc;
       }
     }

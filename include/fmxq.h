@@ -214,8 +214,8 @@ int fmxq_moe_layer(const uint16_t* x, const uint32_t* inds, const uint32_t* w_ga
  *   arena.  That covers, for example, 5120 routed slots at I = 512 or 2048
  *   slots at I = 2048.
  * - A call that needs more scratch returns FMXQ_ERR_SHAPE before anything is
- *   enqueued.  (Long expert runs whose prepared activations do not fit the buffer
- *   run on the shorter-segment kernels instead, to the same tolerance.)
+ *   enqueued.  (A batch whose slots and gated rows fit but whose prepared
+ *   activations do not runs in parts, to the same values.)
  * - Every call on one GPU shares that GPU's buffer, and nothing in it needs to
  *   start at zero.  Calls that overlap on one GPU (concurrent streams, or a
  *   graph replayed while another call runs) race on it and must be serialized

@@ -53,7 +53,7 @@ def _case(gpu, lib, seed, E, T, k, D, I, bits=4):
 def test_noalloc_matches_switch_glu_twice(gpu):
     """A sorted batch (config 3's experts at M = 48: 480 slots, 32-slot windows), then
     a smaller few-slot call (one decode token, 10 slots, no sort) and a small 8-bit
-    call that takes the gather path: each equals fmxq_switch_glu exactly."""
+    call on the segment walk: each equals fmxq_switch_glu exactly."""
     from fastmlx_amd import _lib
 
     lib = _lib.load()
@@ -121,3 +121,43 @@ def test_noalloc_first_call_inside_graph_capture(gpu):
         torch.cuda.synchronize()
         assert np.array_equal(to_np(yg), want), f"replay {rep} differs from fmxq_switch_glu"
         _case(gpu, lib, 30 + rep, E=16, T=3, k=2, D=256, I=256)  # other contents in the buffer
+
+
+@pytest.mark.parametrize("group,E,T,k,D,I", [
+    (32, 8, 1875, 4, 6144, 768),    # 37 MB for the tiles at once, 11.6 MB for the slots
+    (64, 4, 2100, 2, 8192, 256),    # 39 MB
+    (128, 2, 4099, 1, 8192, 512),   # a ragged last part
+])
+def test_noalloc_batch_in_parts(gpu, group, E, T, k, D, I):
+    """Batches whose prepared activations exceed the fixed buffer: answered, with
+    fmxq_switch_glu's bits, and within the oracle's bound."""
+    from fastmlx_amd import _lib, ops
+
+    lib = _lib.load()
+    rng = np.random.default_rng(T)
+    host = [make_quant(rng, (E, I), D, 4, group), make_quant(rng, (E, I), D, 4, group),
+            make_quant(rng, (E, D), I, 4, group)]
+    x, inds = make_x(rng, T, D), topk_uniform(rng, T, E, k)
+    dev = [tuple(to_dev(t, gpu) for t in q) for q in host]
+    dx, di = to_dev(x, gpu), to_dev(inds.astype(np.uint32), gpu)
+    want = ops.switch_glu(dx, di, *dev, group, 4)
+    got = torch.full((T, k, D), 7.0, dtype=torch.bfloat16, device=gpu)
+    announce(f"switch_glu_noalloc in parts: group={group} E={E} T={T} k={k} D={D} I={I}")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    rc = lib.fmxq_switch_glu_noalloc(p(dx), p(di), *(p(t) for q in dev for t in q), p(got), T, k, E,
+                                     D, I, group, 4, None)
+    assert rc == 0, lib.fmxq_last_error()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    sel = np.array([0, T // 2, T - 1])
+    parity.check_switch(to_np(got)[sel], parity.SwitchRef(x, inds, *host, group, 4, token_sel=sel,
+                                                          fused=False), what="in parts")
+
+
+def test_noalloc_gather_path(gpu):
+    """K not a multiple of 256: the general gather kernels."""
+    from fastmlx_amd import _lib
+
+    lib = _lib.load()
+    _case(gpu, lib, 5, E=8, T=40, k=2, D=320, I=320, bits=8)
+    _case(gpu, lib, 6, E=8, T=40, k=2, D=320, I=192)
