@@ -220,33 +220,29 @@ constexpr int64_t kMaxSegmentsGrid = 65535;
 // Scratch of the segmented MoE product in the stream arena: the sorted order,
 // ids and x rows of S slots, the segment table and count, and (SwitchGLU) the
 // h rows of the sorted slots.
-// With max_tiles > 0 also the grouped GEMM's work list and count and (gu_cols > 0)
-// the gate and up rows of its tiles.
+// With max_tiles > 0 also the grouped GEMM's work list and count.
 struct MoeScratch {
   uint32_t *order, *rhs, *lhs, *seg, *nseg;
   uint16_t* h;
   uint32_t *tiles = nullptr, *ntile = nullptr;
-  uint16_t *g = nullptr, *u = nullptr;
   uint8_t* xprep = nullptr;  // with prep > 0: that many bytes for the tiles' x
 };
 struct MoeScratchBytes {
-  size_t ib, sb, hb, tb, gb, pb;
-  MoeScratchBytes(int64_t S, int64_t h_cols, int64_t max_seg, int64_t max_tiles, int64_t gu_cols,
-                  int64_t prep)
+  size_t ib, sb, hb, tb, pb;
+  MoeScratchBytes(int64_t S, int64_t h_cols, int64_t max_seg, int64_t max_tiles, int64_t prep)
       : ib(align_up((size_t)S * sizeof(uint32_t))),
         sb(align_up((size_t)max_seg * 2 * sizeof(uint32_t))),
         hb(align_up((size_t)S * h_cols * sizeof(uint16_t))),
         tb(align_up((size_t)max_tiles * 2 * sizeof(uint32_t))),
-        gb(align_up((size_t)S * gu_cols * sizeof(uint16_t))),
         pb(align_up((size_t)prep)) {}
-  size_t total() const { return 3 * ib + sb + 256 + hb + tb + 256 + 2 * gb + pb; }
+  size_t total() const { return 3 * ib + sb + 256 + hb + tb + 256 + pb; }
 };
 int moe_scratch(hipStream_t s, int64_t S, int64_t h_cols, int64_t max_seg, MoeScratch* m,
-                const char* op, int64_t max_tiles = 0, int64_t gu_cols = 0,
+                const char* op, int64_t max_tiles = 0,
                 const ScratchSource& src = ScratchSource(), int64_t prep = 0,
                 bool* captured = nullptr) {
-  const MoeScratchBytes z(S, h_cols, max_seg, max_tiles, gu_cols, prep);
-  const size_t ib = z.ib, sb = z.sb, hb = z.hb, tb = z.tb, gb = z.gb;
+  const MoeScratchBytes z(S, h_cols, max_seg, max_tiles, prep);
+  const size_t ib = z.ib, sb = z.sb, hb = z.hb, tb = z.tb;
   void* arena = nullptr;
   if (int rc = src.get(s, z.total(), &arena, op, captured)) return rc;
   char* p = static_cast<char*>(arena);
@@ -260,24 +256,18 @@ int moe_scratch(hipStream_t s, int64_t S, int64_t h_cols, int64_t max_seg, MoeSc
   if (max_tiles > 0) {
     m->tiles = reinterpret_cast<uint32_t*>(q);
     m->ntile = reinterpret_cast<uint32_t*>(q + tb);
-    if (gu_cols > 0) {
-      m->g = reinterpret_cast<uint16_t*>(q + tb + 256);
-      m->u = reinterpret_cast<uint16_t*>(q + tb + 256 + gb);
-    }
   }
-  m->xprep = prep > 0 ? reinterpret_cast<uint8_t*>(q + tb + 256 + 2 * gb) : nullptr;
+  m->xprep = prep > 0 ? reinterpret_cast<uint8_t*>(q + tb + 256) : nullptr;
   return FMXQ_OK;
 }
 
-// Expert runs of at least this many slots go to the grouped GEMM (tiles of
-// kGroupedTileRows slots); shorter runs stay on the segment kernels.  Only batches
-// of kGroupedMinSlots or more use it: a grouped block walks all of K, so a few
-// tiles (one 256-slot run: 2 tiles x N/256 blocks) leave the chip idle where the
-// window walk spreads the same run over many blocks.  Batches averaging fewer
-// than kGroupedMinAvgRun slots per expert skip it too: the gate, up and down
-// passes and the silu pass are launched whatever the routing, and with runs that
-// short they rarely find a tile (configuration 3 at M = 512, 10 slots per expert:
-// 252-256 -> 248-250 us per layer).
+// The grouped GEMM serves gather_qmm batches that moe_window keeps from the tiles: expert
+// runs of at least kGroupedMinRun slots, in tiles of kGroupedTileRows; shorter runs stay
+// on the segment kernels.  Only batches of kGroupedMinSlots or more use it: a grouped
+// block walks all of K, so a few tiles (one 256-slot run: 2 tiles x N/256 blocks) leave
+// the chip idle where the window walk spreads the same run over many blocks.  Batches
+// averaging fewer than kGroupedMinAvgRun slots per expert skip it too: it is launched
+// whatever the routing, and with runs that short rarely finds a tile.
 constexpr int64_t kGroupedMinRun = 256;
 constexpr int64_t kGroupedMinSlots = 4096;
 constexpr int64_t kGroupedMinAvgRun = 16;
@@ -565,7 +555,7 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
                                     ? grouped_max_tiles(batch, E)
                                     : 0;
       const int64_t prep = tile ? fmxq::moe_tile_prep_bytes(x_batch * K, bits, group_size) : 0;
-      if (int rc = moe_scratch(s, batch, 0, max_seg, &m, op, max_tiles, 0, ScratchSource(), prep,
+      if (int rc = moe_scratch(s, batch, 0, max_seg, &m, op, max_tiles, ScratchSource(), prep,
                                captured))
         return rc;
       if (int rc = hip_status(fmxq::launch_sort_slots(rhs_indices, batch, lhs_div, E, m.order,
@@ -587,7 +577,7 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
     // Where the stream is being captured and its scratch would have to grow, the next
     // window that needs less, then (formats other than 4 bits in groups of 64, whose
     // general kernels need none) the kernels below.
-    const int first = fmxq::moe_window(batch, E, N, K, N, K, x_batch, bits, group_size);
+    const int first = fmxq::moe_window(batch, E, N, K, x_batch, N, K, x_batch, bits, group_size);
     const int walk = fmxq::moe_walk_window(batch, E);
     for (int window : {first, walk}) {
       const int64_t max_seg = fmxq::moe_max_segments(batch, E, window);
@@ -670,7 +660,7 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
   hipStream_t s = static_cast<hipStream_t>(stream);
   uint32_t* flag = nullptr;
   if (int rc = device_flag(static_cast<hipStream_t>(stream), &flag)) return rc;
-  const int first = fmxq::moe_window(S, E, I, D, D, I, std::max(S, T), bits, group_size);
+  const int first = fmxq::moe_window(S, E, I, D, T, D, I, S, bits, group_size);
   const int walk = fmxq::moe_walk_window(S, E);
   // The tiles keep a prepared copy of x, then of h.
   auto prep_bytes = [&](int64_t nt) {
@@ -690,7 +680,7 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
     // slots skip the sort: each is its own segment, h stays in slot order.
     auto unsorted = [&](bool* captured) -> int {
       MoeScratch m;
-      if (int rc = moe_scratch(s, S, I, 1, &m, op, 0, 0, src, 0, captured)) return rc;
+      if (int rc = moe_scratch(s, S, I, 1, &m, op, 0, src, 0, captured)) return rc;
       fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
                        nullptr, m.h, nullptr, S, I, D, E, T, flag, group_size, bits, topk};
       if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, 16, S, s), "switch_glu: gate/up"))
@@ -706,20 +696,10 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
       const uint16_t* const xt = x + t0 * D;
       uint16_t* const yt = out + t0 * topk * D;
       const bool tile = window == fmxq::kMoeTileRows;
-      // Long expert runs (>= kGroupedMinRun slots) go to the grouped GEMM: gate and
-      // up into g and u, silu * up into their h rows, then down.
-      const int64_t max_tiles =
-          !tile && fmxq::qmm_grouped_supported(I, D, T, bits, group_size) &&
-                  fmxq::qmm_grouped_supported(D, I, S, bits, group_size)
-              ? grouped_max_tiles(S, E)
-              : 0;
-      if (int rc = moe_scratch(s, S, I, max_seg, &m, op, max_tiles, max_tiles ? I : 0, src,
-                               tile ? prep_bytes(nt) : 0, captured))
+      if (int rc = moe_scratch(s, S, I, max_seg, &m, op, 0, src, tile ? prep_bytes(nt) : 0, captured))
         return rc;
       if (int rc = hip_status(fmxq::launch_sort_slots(inds + t0 * topk, S, topk, E, m.order, m.rhs, m.lhs, s,
-                                                      nullptr, m.seg, m.nseg, window, m.tiles,
-                                                      m.ntile, (int)kGroupedMinRun,
-                                                      fmxq::kGroupedTileRows),
+                                                      nullptr, m.seg, m.nseg, window),
                               "switch_glu: sort"))
         return rc;
       fmxq::MoeArgs gu{xt, m.lhs, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, m.rhs, m.seg,
@@ -728,30 +708,10 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
       if (int rc = hip_status(fmxq::launch_moe_qmvs(gu, 2, window, max_seg, s),
                               "switch_glu: gate/up"))
         return rc;
-      if (max_tiles) {
-        const fmxq::QmmArgs gg = grouped_args(xt, w_gate, s_gate, b_gate, m.g, I, D, bits,
-                                              group_size, m, m.lhs, nullptr, T, flag);
-        if (int rc = hip_status(fmxq::launch_qmm_grouped(gg, max_tiles, s), "switch_glu: gate"))
-          return rc;
-        const fmxq::QmmArgs gup = grouped_args(xt, w_up, s_up, b_up, m.u, I, D, bits, group_size,
-                                               m, m.lhs, nullptr, T, flag);
-        if (int rc = hip_status(fmxq::launch_qmm_grouped(gup, max_tiles, s), "switch_glu: up"))
-          return rc;
-        if (int rc = hip_status(fmxq::launch_silu_mul_tiles(m.g, m.u, m.h, m.tiles, m.ntile,
-                                                            max_tiles, fmxq::kGroupedTileRows, I,
-                                                            s),
-                                "switch_glu: silu"))
-          return rc;
-      }
       fmxq::MoeArgs dn{m.h, nullptr, {w_down, nullptr}, {s_down, nullptr}, {b_down, nullptr},
                        m.rhs, m.seg, m.nseg, yt, m.order, S, D, I, E, S, flag, group_size, bits};
       dn.xprep = m.xprep;
-      if (int rc = hip_status(fmxq::launch_moe_qmvs(dn, 1, window, max_seg, s), "switch_glu: down"))
-        return rc;
-      if (!max_tiles) return FMXQ_OK;
-      const fmxq::QmmArgs gd = grouped_args(m.h, w_down, s_down, b_down, yt, D, I, bits,
-                                            group_size, m, nullptr, m.order, S, flag);
-      return hip_status(fmxq::launch_qmm_grouped(gd, max_tiles, s), "switch_glu: down");
+      return hip_status(fmxq::launch_moe_qmvs(dn, 1, window, max_seg, s), "switch_glu: down");
     };
     if (S <= fmxq::kMoeUnsortedMaxSlots) {
       bool captured = false;
@@ -765,10 +725,10 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
         // otherwise).  The whole batch's h rows and slots have to fit all the same.
         const int64_t walk_seg = fmxq::moe_max_segments(S, E, walk);
         void* unused = nullptr;
-        if (int rc = src.get(s, MoeScratchBytes(S, I, walk_seg, 0, 0, 0).total(), &unused, op)) return rc;
+        if (int rc = src.get(s, MoeScratchBytes(S, I, walk_seg, 0, 0).total(), &unused, op)) return rc;
         int64_t parts = 1, nt = T;
         auto bytes = [&](int64_t n) {
-          return MoeScratchBytes(n * topk, I, fmxq::moe_max_segments(n * topk, E, first), 0, 0,
+          return MoeScratchBytes(n * topk, I, fmxq::moe_max_segments(n * topk, E, first), 0,
                                  prep_bytes(n)).total();
         };
         while (nt > 1 && bytes(nt) > src.fixed_bytes) nt = (T + parts) / (parts + 1), ++parts;
@@ -887,7 +847,7 @@ extern "C" int fmxq_switch_glu_combine(
     if (int rc = device_flag(static_cast<hipStream_t>(stream), &flag)) return rc;
     MoeScratch m;
     bool captured = false;
-    const int rc = moe_scratch(s, S, I, 1, &m, op, 0, 0, ScratchSource(), 0, &captured);
+    const int rc = moe_scratch(s, S, I, 1, &m, op, 0, ScratchSource(), 0, &captured);
     if (rc && !captured) return rc;
     if (!rc) {
       fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
@@ -954,7 +914,7 @@ extern "C" int fmxq_moe_layer(
     if (int rc = device_flag(s, &flag)) return rc;
     MoeScratch m;
     bool captured = false;
-    const int rc = moe_scratch(s, S + T, I, 1, &m, op, 0, 0, ScratchSource(), 0, &captured);
+    const int rc = moe_scratch(s, S + T, I, 1, &m, op, 0, ScratchSource(), 0, &captured);
     if (rc && !captured) return rc;
     if (!rc) {
       fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
@@ -975,13 +935,13 @@ extern "C" int fmxq_moe_layer(
                         "moe_layer: down/combine");
     }
   }
-  // Sorted batches below the grouped GEMM's floor: the shared expert joins the
-  // sort as expert id E with one slot per token (after the S routed slots), so its
-  // segments ride in the routed gate/up and down launches; the rows land in the
-  // arena's slot 1, routed then shared, and the combine reads both.
+  // Sorted batches: the shared expert joins the sort as expert id E with one slot per
+  // token (after the S routed slots), so its segments ride in the routed gate/up and
+  // down launches; the rows land in the arena's slot 1, routed then shared, and the
+  // combine reads both.
   {
     const int64_t Sa = S + T;
-    const int window = fmxq::moe_window(Sa, E + 1, I, D, D, I, Sa, bits, group_size);
+    const int window = fmxq::moe_window(Sa, E + 1, I, D, T, D, I, Sa, bits, group_size);
     const int64_t max_seg = fmxq::moe_max_segments(Sa, E + 1, window);
     auto layer = [&](const MoeScratch& m, uint16_t* y) -> int {
       uint32_t* flag = nullptr;
@@ -1018,7 +978,6 @@ extern "C" int fmxq_moe_layer(
                         "moe_layer: combine");
     };
     if (!fmxq::moe_combine_unsorted(S, E) &&
-        (window == fmxq::kMoeTileRows || grouped_max_tiles(S, E) == 0) &&
         E + 1 <= kSortMaxExperts && max_seg <= kMaxSegmentsGrid &&
         fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
         fmxq::moe_qmvs_supported(D, I, S + T, bits, group_size) && aligned16(s_gate) &&
@@ -1032,7 +991,7 @@ extern "C" int fmxq_moe_layer(
               : 0;
       void* rows = nullptr;
       bool captured = false;
-      int rc = moe_scratch(s, Sa, I, max_seg, &m, op, 0, 0, ScratchSource(), prep, &captured);
+      int rc = moe_scratch(s, Sa, I, max_seg, &m, op, 0, ScratchSource(), prep, &captured);
       if (!rc)
         rc = stream_arena(s, align_up((size_t)Sa * D * sizeof(uint16_t)), &rows, op, 1, &captured);
       if (rc && !captured) return rc;

@@ -200,9 +200,6 @@ hipError_t launch_sort_slots(const uint32_t* inds, int64_t S, int64_t lhs_div, i
                              uint32_t* seg = nullptr, uint32_t* nseg = nullptr, int window = 16,
                              uint32_t* tiles = nullptr, uint32_t* ntile = nullptr,
                              int long_min = 0, int tile_rows = 0, int64_t sh_T = 0);
-hipError_t launch_silu_mul_tiles(const uint16_t* g, const uint16_t* u, uint16_t* h,
-                                 const uint32_t* tiles, const uint32_t* ntile, int64_t max_tiles,
-                                 int64_t tile_rows, int64_t n, hipStream_t stream);
 hipError_t launch_silu_mul(const uint16_t* g, const uint16_t* u, uint16_t* h, int64_t n,
                            hipStream_t stream);
 hipError_t launch_moe_combine(const uint16_t* y, const uint16_t* w, const uint16_t* shared,
@@ -304,11 +301,11 @@ inline int64_t moe_tile_prep_bytes(int64_t n, int bits, int group_size) {
 }
 bool moe_qmvs_supported(int64_t N, int64_t K, int64_t x_rows, int bits, int group_size);
 // Slots per segment of a sorted batch of S slots over E experts, for products of N1 x
-// K1 and then N2 x K2 per slot whose x has at most x_rows rows: 16 or 32 for the walk,
+// K1 and then N2 x K2 per slot whose x has rows1 and rows2 rows: 16 or 32 for the walk,
 // kMoeTileRows for the tiles.
 int moe_walk_window(int64_t S, int64_t E);
-int moe_window(int64_t S, int64_t E, int64_t N1, int64_t K1, int64_t N2, int64_t K2,
-               int64_t x_rows, int bits, int group_size);
+int moe_window(int64_t S, int64_t E, int64_t N1, int64_t K1, int64_t rows1, int64_t N2, int64_t K2,
+               int64_t rows2, int bits, int group_size);
 int64_t moe_max_segments(int64_t S, int64_t E, int window);
 hipError_t launch_moe_qmvs(const MoeArgs& a, int nmat, int window, int64_t max_seg,
                            hipStream_t stream);

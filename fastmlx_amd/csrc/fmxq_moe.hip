@@ -275,49 +275,6 @@ hipError_t launch_sort_slots(const uint32_t* inds, int64_t S, int64_t lhs_div, i
   return hipGetLastError();
 }
 
-// h rows of the grouped-GEMM tiles: h = silu(g) * u with the op chain's roundings
-// (silu_mul_kernel's arithmetic).  Grid (column blocks, tile bound); a block
-// covers 256 x 8 values of one tile: rows start .. start + len, n cols.
-__global__ __launch_bounds__(256) void silu_mul_tiles_kernel(const uint16_t* __restrict__ g,
-                                                             const uint16_t* __restrict__ u,
-                                                             uint16_t* __restrict__ h,
-                                                             const uint32_t* __restrict__ tiles,
-                                                             const uint32_t* __restrict__ ntile,
-                                                             int64_t n) {
-  const int64_t t = blockIdx.y;
-  if (t >= (int64_t)*ntile) return;
-  const int64_t start = tiles[2 * t], len = tiles[2 * t + 1];
-  const int64_t n8 = n / 8, items = len * n8;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < items;
-       i += (int64_t)gridDim.x * 256) {
-    const int64_t r = start + i / n8, c = i % n8;
-    const u32x4 gv = reinterpret_cast<const u32x4*>(g + r * n)[c];
-    const u32x4 uv = reinterpret_cast<const u32x4*>(u + r * n)[c];
-    u32x4 o;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float g0 = bf16_lo(gv[j]), g1 = bf16_hi(gv[j]);
-      const float s0 = r16(1.f / (1.f + __expf(-g0))), s1 = r16(1.f / (1.f + __expf(-g1)));
-      const float h0 = r16(r16(g0 * s0) * bf16_lo(uv[j]));
-      const float h1 = r16(r16(g1 * s1) * bf16_hi(uv[j]));
-      o[j] = f32_to_bf16_rne(h0) | (f32_to_bf16_rne(h1) << 16);
-    }
-    reinterpret_cast<u32x4*>(h + r * n)[c] = o;
-  }
-}
-
-hipError_t launch_silu_mul_tiles(const uint16_t* g, const uint16_t* u, uint16_t* h,
-                                 const uint32_t* tiles, const uint32_t* ntile, int64_t max_tiles,
-                                 int64_t tile_rows, int64_t n, hipStream_t stream) {
-  if (max_tiles <= 0) return hipSuccess;
-  if (n % 8 != 0) return hipErrorInvalidValue;
-  const int64_t per_tile = tile_rows * (n / 8);
-  dim3 grid((unsigned)((per_tile + 255) / 256 < 64 ? (per_tile + 255) / 256 : 64),
-            (unsigned)max_tiles);
-  silu_mul_tiles_kernel<<<grid, 256, 0, stream>>>(g, u, h, tiles, ntile, n);
-  return hipGetLastError();
-}
-
 hipError_t launch_silu_mul(const uint16_t* g, const uint16_t* u, uint16_t* h, int64_t n,
                            hipStream_t stream) {
   const int64_t n8 = n / 8;

@@ -637,17 +637,19 @@ int moe_walk_window(int64_t S, int64_t E) { return S >= 4 * E ? 32 : 16; }
 // (36) 2705 / 2189; 64 experts x 1536, K = 3072, top-6: 250 tokens (23, 1500 slots)
 // 186 / 196, 600 (56) 340 / 254, 900 (84) in groups of 32 688 / 498; 16 experts x 1792,
 // top-8, 1407 tokens (703) 1021 / 662; 16 experts x 1024, K = 2048, top-4: 200 tokens
-// (50, 264 blocks) 69 / 72.  Batches the tiles do not take (outputs not a multiple of
-// 32, x of 2^31 bytes, the allocation-free call's scratch) keep the walk and, for their
-// long runs, the grouped GEMM.
-int moe_window(int64_t S, int64_t E, int64_t N1, int64_t K1, int64_t N2, int64_t K2,
-               int64_t x_rows, int bits, int group_size) {
-  const int64_t kmax = K1 > K2 ? K1 : K2;
+// (50, 264 blocks) 69 / 72.  There is no upper end: against the grouped GEMM that runs of
+// 256 and more had, SwitchGLU (us) of 2 experts x 2048, K = 2048, top-2, 1024 tokens (1024
+// slots per expert) 151 / 117, 4 x 4096, K = 4096, 4096 tokens (2048) 1485 / 1085, 8 x
+// 1024, K = 2048, 16384 tokens (4096) 805 / 669, 2 x 2048, top-1, 8192 tokens (4096) 449 /
+// 362; one product by gather_qmm 1.07 to 1.32 times.  Batches the tiles do not take
+// (outputs not a multiple of 32, x of 2^31 bytes) keep the walk.
+int moe_window(int64_t S, int64_t E, int64_t N1, int64_t K1, int64_t rows1, int64_t N2, int64_t K2,
+               int64_t rows2, int bits, int group_size) {
   const int64_t blocks = (E + S / kMoeTileRows) * ((N1 + 127) / 128);
   if (S >= 16 * E && (S >= 4096 || (S >= 48 * E && blocks >= 512)) && N1 % 32 == 0 && N2 % 32 == 0 &&
-      x_rows * kmax * 2 < (int64_t(1) << 31) &&
-      moe_qmvs_supported(N1, K1, x_rows, bits, group_size) &&
-      moe_qmvs_supported(N2, K2, x_rows, bits, group_size))
+      rows1 * K1 * 2 < (int64_t(1) << 31) && rows2 * K2 * 2 < (int64_t(1) << 31) &&
+      moe_qmvs_supported(N1, K1, rows1, bits, group_size) &&
+      moe_qmvs_supported(N2, K2, rows2, bits, group_size))
     return kMoeTileRows;
   return moe_walk_window(S, E);
 }

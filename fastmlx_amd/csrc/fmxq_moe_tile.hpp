@@ -495,7 +495,7 @@ __global__ __launch_bounds__(256) void tile_prep_kernel(const uint16_t* __restri
         u32x2{hi | (mid << 16), lo};
 }
 
-// Grid: (column tiles, segment bound).  The caller checks the sizes (moe_tile_supported):
+// Grid: (column tiles, segment bound).  The caller checks the sizes (moe_window):
 // x and each expert's matrix below 2^31 bytes, fewer than 2^31 rows.
 template <int NMAT, int BITS, int GS>
 __global__ __launch_bounds__(kTileWaves * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_tile_kernel(

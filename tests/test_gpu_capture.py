@@ -123,8 +123,8 @@ def test_gather_qmm_captured_within_walk_scratch(gpu, oracle):
 
 
 def test_switch_glu_captured_within_walk_scratch(gpu, oracle):
-    """The same for SwitchGLU: 9.8 MB from 300 slots of I = 16384, 6.5 MB for the walk of 4200
-    slots, 11.8 MB for its tiles."""
+    """The same for SwitchGLU: 9.8 MB from 300 slots of I = 16384, 2.3 MB for the walk of 4200
+    slots, 11.4 MB for its tiles."""
     from fastmlx_amd import ops
     from synth import topk_uniform
 

@@ -510,12 +510,13 @@ def test_switch_glu_many_slots_per_expert_long_rows(gpu, oracle):
     _check(got, x, inds, gate, up, down)
 
 
-# --- long expert runs (>= 256 slots, batches of >= 4096 slots): the grouped GEMM ---
+# --- long expert runs: SwitchGLU on the tiles; the grouped GEMM (>= 256 slots, batches of
+# >= 4096 slots) where gather_qmm's outputs are not a multiple of 32 ---
 
 @pytest.mark.parametrize("E,T,k,D,I", [
-    (2, 2100, 2, 256, 256),    # two runs of 2100 slots: 16 full tiles and a partial each
+    (2, 2100, 2, 256, 256),    # two runs of 2100 slots: full tiles and a partial each
     (3, 2100, 2, 256, 512),    # three runs of ~1400
-    (24, 1024, 4, 256, 256),   # Zipf: runs of 838 .. 281 grouped, 239 and below on the walk
+    (24, 1024, 4, 256, 256),   # Zipf: runs from 838 down
     (2, 8200, 2, 256, 256),    # 16400 slots: more than the sort's LDS staging holds
 ])
 def test_switch_glu_long_runs(gpu, oracle, E, T, k, D, I):
@@ -1160,3 +1161,22 @@ def test_tiles_switch_glu_nonfinite_rows(gpu, oracle, bits, group):
     rest = torch.ones(T, dtype=torch.bool)
     rest[3:6] = False
     assert torch.equal(got[rest], plain[rest])
+
+
+def test_switch_glu_large_activations(gpu):
+    """T x D and S x I below 2^31 bytes, S x D above: on the tiles, as each half of the
+    tokens is by itself, so with the same bits."""
+    from fastmlx_amd import ops
+
+    E, T, k, D, I = 4, 33000, 2, 16384, 256
+    gen = torch.Generator(device=gpu).manual_seed(1)
+    x = torch.empty(T, D, device=gpu, dtype=torch.bfloat16).normal_(generator=gen)
+    inds = torch.rand(T, E, device=gpu, generator=gen).topk(k, -1).indices.int()
+    rng = np.random.default_rng(2)
+    stacks = [tuple(to_dev(t, gpu) for t in make_quant(rng, lead, K, 4, 64))
+              for lead, K in (((E, I), D), ((E, I), D), ((E, D), I))]
+    announce(f"switch_glu with {T * k * D * 2} bytes of outputs")
+    got = ops.switch_glu(x, inds, *stacks)
+    for at in (slice(0, T // 2), slice(T // 2, T)):
+        half = ops.switch_glu(x[at].contiguous(), inds[at].contiguous(), *stacks)
+        assert torch.equal(got[at], half)
