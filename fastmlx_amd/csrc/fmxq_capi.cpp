@@ -577,8 +577,14 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
     // Where the stream is being captured and its scratch would have to grow, the next
     // window that needs less, then (formats other than 4 bits in groups of 64, whose
     // general kernels need none) the kernels below.
-    const int first = fmxq::moe_window(batch, E, N, K, x_batch, N, K, x_batch, bits, group_size);
+    // The tiles prepare every row of x, read or not, so they take an x of up to twice as
+    // many rows as the batch has items (x rows / items 1, 2, 4, 16; walk against tiles,
+    // us: 8192 items, 4 experts of 2048 x 2048 160 / 142, 157 / 152, 159 / 190, 160 / 368;
+    // 4200 items, 8 of 1024 x 4096 127 / 105, 128 / 118, 127 / 155, 127 / 341).
     const int walk = fmxq::moe_walk_window(batch, E);
+    const int first = x_batch <= 2 * batch
+                          ? fmxq::moe_window(batch, E, N, K, x_batch, N, K, x_batch, bits, group_size)
+                          : walk;
     for (int window : {first, walk}) {
       const int64_t max_seg = fmxq::moe_max_segments(batch, E, window);
       if (max_seg > kMaxSegmentsGrid) continue;

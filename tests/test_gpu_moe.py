@@ -4,6 +4,8 @@ Shapes mirror the reference's own SwitchGLU tests (compute/models/switch_glu_tes
 5 experts, d=64, h=128, group 64 int4 for the unsorted branch with 2x3 slots; 8
 experts with 32x2 = 64 slots for the sorted branch) and BASELINE configs 3 and 4.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -1180,3 +1182,31 @@ def test_switch_glu_large_activations(gpu):
     for at in (slice(0, T // 2), slice(T // 2, T)):
         half = ops.switch_glu(x[at].contiguous(), inds[at].contiguous(), *stacks)
         assert torch.equal(got[at], half)
+
+
+def test_gather_qmm_few_items_of_a_large_x(gpu, oracle):
+    """A batch that reads 4200 of 200000 rows of x (205 MB) keeps no copy of x."""
+    from fastmlx_amd import ops
+
+    rng = np.random.default_rng(8)
+    E, S, xb, N, K = 4, 4200, 200000, 64, 512
+    q = make_quant(rng, (E, N), K, 4, 64)
+    x = torch.empty(xb, 1, K, device=gpu, dtype=torch.bfloat16).normal_()
+    rhs = rng.integers(0, E, size=S).astype(np.uint32)
+    lhs = rng.integers(0, xb, size=S).astype(np.uint32)
+    dev = [to_dev(t, gpu) for t in (*q, rhs, lhs)]
+    y = torch.empty(S, 1, N, device=gpu, dtype=torch.bfloat16)
+    announce(f"gather_qmm of {S} items over {xb} rows of x")
+    hip = ctypes.CDLL("libamdhip64.so")
+    s = ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(s), 1) == 0  # its scratch starts empty
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    with torch.cuda.stream(torch.cuda.ExternalStream(s.value)):
+        ops.gather_qmm(x, *dev, 1, True, 64, 4, False, y)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 50 << 20
+    sel = rng.choice(S, size=100, replace=False)
+    rows = to_np(x[torch.from_numpy(lhs[sel].astype(np.int64)).to(gpu), 0].contiguous())
+    ref = parity.gather_refs(rows, *q, np.arange(100, dtype=np.int32), rhs[sel].astype(np.int32))
+    parity.check_dense(to_np(y).reshape(S, N)[sel], ref, what="gather_qmm")
