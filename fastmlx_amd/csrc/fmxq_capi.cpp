@@ -216,6 +216,9 @@ size_t align_up(size_t v) { return (v + 255) & ~(size_t)255; }
 constexpr int64_t kSortMaxExperts = 16384;
 // Segments run along the grid's y axis.
 constexpr int64_t kMaxSegmentsGrid = 65535;
+// Weight bytes the shared expert of an unsorted batch may read inside the routed
+// kernels (fmxq_moe_layer).
+constexpr int64_t kMoeSharedInMaxBytes = 192 << 20;
 
 // Scratch of the segmented MoE product in the stream arena: the sorted order,
 // ids and x rows of S slots, the segment table and count, and (SwitchGLU) the
@@ -906,12 +909,17 @@ extern "C" int fmxq_moe_layer(
   hipStream_t s = static_cast<hipStream_t>(stream);
   // Unsorted batches (decode): the shared expert rides along as one more gate/up
   // segment per token and one more wave of each down/combine block, two launches for
-  // the layer.  Its weights are then read once per token, from L2 after the first,
-  // which costs less than the four launches of a one-expert SwitchGLU up to the most
-  // slots an unsorted batch has (512 experts of 512 columns, top-10, K = 2048: 2 / 12 /
-  // 25 tokens, router included, 32.8 / 68.6 / 115.8 -> 23.2 / 56.5 / 94.0 us, about
-  // 3.5 us of it the router's own gain).
+  // the layer.  Its weights are then read once per token, from L2 after the first; on
+  // its own it is a one-expert SwitchGLU, four launches, which reads them once per
+  // token too up to 16 tokens and once in all beyond.  So past 16 tokens it rides along
+  // while these reads stay below kMoeSharedInMaxBytes (own / along, us a layer: 512
+  // experts x 512, K = 2048, top-10 at 2 / 24 tokens 19 / 13 and 97 / 80, top-1 at 96 /
+  // 128 / 192 tokens (151, 201 and 302 MB) 59 / 50, 69 / 65 and 89 / 95; 256 x 2048, K =
+  // 4096, top-1 at 16 / 24 / 128 tokens 83 / 78, 91 / 113 (302 MB) and 358 / 563; K = 7168,
+  // top-4 at 16 / 24 tokens 341 / 340 and 437 / 506 (528 MB)).
+  const int64_t shared_bytes = 3 * D * I * bits / 8;
   if (topk <= 15 && fmxq::moe_combine_unsorted(S, E) && D >= 2048 && D <= 16384 &&
+      (T <= 16 || T * shared_bytes <= kMoeSharedInMaxBytes) &&
       fmxq::moe_down_combine_supported(T, topk, D, I, bits, group_size) &&
       fmxq::moe_qmvs_supported(I, D, T, bits, group_size) && aligned16(s_gate) &&
       aligned16(b_gate) && aligned16(s_up) && aligned16(b_up) && aligned16(ss_gate) &&

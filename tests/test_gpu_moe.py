@@ -774,11 +774,10 @@ def test_one_token_layer_back_to_back(gpu, oracle):
 def test_moe_layer_shared_expert_c4(gpu, oracle, M):
     """Configuration 4 with its shared expert computed inside the call
     (deepseekv3_forward.go:436-440: routed sum + mlp(x)), up to M=256, the largest
-    token count the bench times.  One token runs the
-    shared expert as one more gate/up segment and one more down/combine wave; three
-    tokens (24 slots, few sharing an expert) run it as a one-expert SwitchGLU first;
-    sorted batches (32 and 256 tokens) sort it in as expert E, one slot per token,
-    inside the routed launches.  Checked element by element against the oracle's
+    token count the bench times.  One token and three (24 slots, few sharing an expert)
+    run the shared expert as one more gate/up segment per token and one more
+    down/combine wave; sorted batches (32 and 256 tokens) sort it in as expert E, one
+    slot per token, inside the routed launches.  Checked element by element against the oracle's
     routed experts and shared MLP."""
     from fastmlx_amd import ops
 
@@ -806,14 +805,41 @@ def test_moe_layer_shared_expert_c4(gpu, oracle, M):
                          shared=(sv[:, 0], sa[:, 0]), what=f"moe_layer c4 M={M}")
 
 
+@pytest.mark.parametrize("T", [16, 100, 192, 256])
+def test_moe_layer_shared_expert_one_pick(gpu, oracle, T):
+    """Unsorted batches of one slot per token (512 experts): the shared expert in the routed
+    kernels up to 16 tokens and while its reads stay below the limit (157 MB at 100
+    tokens), a one-expert SwitchGLU first beyond (302 MB at 192)."""
+    from fastmlx_amd import ops
+
+    (gate, up, down), dstack, shared, dshared = _layer_weights(gpu, "c3")
+    rng = np.random.default_rng(970 + T)
+    E, D = gate[0].shape[0], down[0].shape[1]
+    inds = topk_uniform(rng, T, E, 1)
+    w16 = oracle.f32_to_bf16(np.ones((T, 1), dtype=np.float32))
+    x = make_x(rng, T, D)
+    announce(f"moe_layer top-1 T={T} E={E} + shared expert")
+    out = ops.moe_layer(to_dev(x, gpu), to_dev(inds.astype(np.uint32), gpu), *dstack,
+                        to_dev(w16, gpu), dshared)
+    torch.cuda.synchronize()
+    sel = np.array([0, T // 2, T - 1])
+    sref = parity.SwitchRef(x, inds, gate, up, down, token_sel=sel, fused=False)
+    near = sref.refs[0]
+    ssref = parity.SwitchRef(x, np.zeros((T, 1), dtype=np.int32), *shared, token_sel=sel, fused=False)
+    sv = ssref.refs[0]
+    sa = parity.switch_bound(sv, sv, ssref.hscale)
+    parity.combine_check(to_np(out)[sel], near, parity.switch_bound(near, near, sref.hscale), w16[sel],
+                         shared=(sv[:, 0], sa[:, 0]), what=f"moe_layer top-1 T={T}")
+
+
 @pytest.mark.parametrize("T,E,D,k", [(1, 300, 2048, 10), (2, 300, 2048, 10),
                                      (1, 64, 2048, 16), (1, 40, 512, 6),
                                      (24, 32, 2048, 6), (40, 16, 512, 4)])
 def test_moe_layer_gated_shared_expert(gpu, oracle, T, E, D, k):
     """A Qwen3-Next-style layer (qwen3next_forward.go:519-524): the shared expert's
-    output scaled by sigmoid(shared_gate) before it is added.  One token with up
-    to 15 slots and D >= 2048 runs fused; two tokens, 16 slots (a block would need
-    17 waves) and D = 512 (below the GEMV form's depth) run the one-expert
+    output scaled by sigmoid(shared_gate) before it is added.  One and two tokens with
+    up to 15 picks each and D >= 2048 run fused; 16 picks (a block would need 17
+    waves) and D = 512 (below the GEMV form's depth) run the one-expert
     SwitchGLU first; 24 and 40 tokens over few experts sort the shared expert in
     as expert E (16- and 32-slot segments; D = 512 walks its down projection with
     every load issued up front)."""
