@@ -812,9 +812,11 @@ def test_moe_layer_shared_expert_one_pick(gpu, oracle, T):
     tokens), a one-expert SwitchGLU first beyond (302 MB at 192)."""
     from fastmlx_amd import ops
 
-    (gate, up, down), dstack, shared, dshared = _layer_weights(gpu, "c3")
+    (gate, up, down), dstack, _, _ = _layer_weights(gpu, "c3")
     rng = np.random.default_rng(970 + T)
     E, D = gate[0].shape[0], down[0].shape[1]
+    shared = _stack(rng, 1, D, 512)
+    dshared = [tuple(to_dev(t, gpu) for t in q) for q in shared]
     inds = topk_uniform(rng, T, E, 1)
     w16 = oracle.f32_to_bf16(np.ones((T, 1), dtype=np.float32))
     x = make_x(rng, T, D)
