@@ -2,7 +2,8 @@
 
 ``python -m fastmlx_amd.build`` or ``fastmlx_amd.build.build()``.  Objects go to
 ``fastmlx_amd/_build/``; the shared library lands next to this file so it
-travels with the source tree, and so does ``_fast.so``, the torch wrappers' call path.
+travels with the source tree, and so does ``_fast``, the torch wrappers' call path, where
+torch is installed.
 ``--diag`` (``build_diag()``) also builds the
 time-line diagnostic program ``diag/qmv1_timeline``.
 """
@@ -73,20 +74,36 @@ def build_diag(verbose: bool = True) -> str:
     return TIMELINE
 
 
-FAST = os.path.join(HERE, "_fast.so")
+# Tagged with the interpreter's ABI, so another Python in the same tree does not load it.
+FAST = os.path.join(HERE, "_fast" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 
-def build_fast(verbose: bool = True) -> str:
+def _cxx() -> str | None:
+    rocm = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin", "clang++")
+    return shutil.which("g++") or shutil.which("clang++") or (rocm if os.path.exists(rocm) else None)
+
+
+def build_fast(verbose: bool = True) -> str | None:
     """The torch wrappers' call path in C++ (ext/fmxq_fast.cpp), a CPython module linked
-    against torch and the libfmxq.so next to it."""
-    torch_dir = list(importlib.util.find_spec("torch").submodule_search_locations)[0]
+    against torch and the libfmxq.so next to it.  The wrappers run without it, so where
+    torch for ROCm or a C++ compiler is missing it is left out and None returned."""
+    spec = importlib.util.find_spec("torch")
+    torch_dir = list(spec.submodule_search_locations)[0] if spec else ""
+    lib = os.path.join(torch_dir, "lib")
+    cxx = _cxx()
+    old = os.path.join(HERE, "_fast.so")  # the name without a tag, from an earlier build
+    if os.path.exists(old):
+        os.remove(old)
+    if not cxx or not os.path.exists(os.path.join(lib, "libc10_hip.so")):
+        if verbose:
+            print("skipped " + FAST + ": " + ("no torch for ROCm" if cxx else "no C++ compiler"))
+        return None
     rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
     inc = [os.path.join(torch_dir, "include"), sysconfig.get_paths()["include"],
            os.path.join(torch_dir, "include", "torch", "csrc", "api", "include"),
            os.path.join(rocm, "include")]
-    lib = os.path.join(torch_dir, "lib")
     tmp = FAST + ".tmp"
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
            "-DUSE_ROCM=1", *(a for d in inc for a in ("-isystem", d)),
            os.path.join(HERE, "ext", "fmxq_fast.cpp"), "-o", tmp, f"-L{lib}", "-lc10", "-lc10_hip",
            "-ltorch_cpu", "-ltorch_python", f"-L{HERE}", "-l:libfmxq.so", "-Wl,-rpath,$ORIGIN",
