@@ -8,8 +8,10 @@
 //
 // A function returns None, with nothing enqueued, for anything but the plain case: an
 // argument that ops.py would refuse, a tensor subclass, a functorch wrapper, an active
-// dispatch or function mode, sizes of zero, or a nonzero status of the library.  ops.py
-// then runs its own path, which raises the error or handles the call.
+// dispatch or function mode, or sizes of zero.  ops.py then runs its own path, which
+// raises the error or handles the call.  A nonzero status of the library is raised from
+// here, as ops.py raises it: a second attempt would enqueue again what the first had
+// launched, and an error of the device, reported once, would be lost.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -113,14 +115,20 @@ void* stream_of(const at::Tensor& t) {
   return c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
 
-// Run f() without the GIL; its status 0 means enqueued.
+// Run f() without the GIL; its status 0 means enqueued, another sets the Python error
+// that fastmlx_amd._lib.check raises for it.
 template <class F>
 bool enqueue(F&& f) {
   int rc;
   Py_BEGIN_ALLOW_THREADS;
   rc = f();
   Py_END_ALLOW_THREADS;
-  return rc == FMXQ_OK;
+  if (rc == FMXQ_OK) return true;
+  if (PyObject* lib = PyImport_ImportModule("fastmlx_amd._lib")) {
+    Py_XDECREF(PyObject_CallMethod(lib, "check", "i", rc));
+    Py_DECREF(lib);
+  }
+  return false;
 }
 
 // C++ exceptions (out of memory in an allocation) leave through Python's path, which
@@ -129,10 +137,10 @@ template <class F>
 PyObject* guarded(F&& f) {
   try {
     PyObject* r = f();
-    if (r) return r;
+    if (r || PyErr_Occurred()) return r;
   } catch (...) {
+    PyErr_Clear();
   }
-  PyErr_Clear();
   Py_RETURN_NONE;
 }
 

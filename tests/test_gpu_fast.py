@@ -108,3 +108,105 @@ def test_fast_path_refusals(gpu):
     param = torch.nn.Parameter(x[:, :256].contiguous())
     y = ops.quantized_matmul(param, w, s, b)
     assert not y.requires_grad and torch.equal(y, ops.quantized_matmul(param.data, w, s, b))
+
+
+class _Recorder:
+    """fastmlx_amd._fast with a note of what each call returned."""
+
+    def __init__(self, mod):
+        self.mod, self.calls = mod, []
+
+    def __getattr__(self, name):
+        def call(*args):
+            r = getattr(self.mod, name)(*args)
+            self.calls.append((name, r is not None))
+            return r
+        return call
+
+
+NAMES = {"quantized_matmul", "dequantize", "quantize", "moe_layer", "route_softmax_topk",
+         "route_group_topk"}
+
+
+@pytest.mark.parametrize("mode", ["plain", "inference", "graph"])
+def test_fast_path_answers_plain_calls(gpu, monkeypatch, mode):
+    """Every function of the module answers the plain calls itself."""
+    from fastmlx_amd import ops
+
+    announce(f"fast path answers {mode}")
+    run = _calls(gpu, 4, 64)
+    run()
+    rec = _Recorder(ops._fast)
+    monkeypatch.setattr(ops, "_fast", rec)
+    if mode == "plain":
+        run()
+    elif mode == "inference":
+        with torch.inference_mode():
+            run()
+    else:
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            run()
+        stream.synchronize()
+        rec.calls.clear()
+        with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=stream):
+            run()
+    torch.cuda.synchronize()
+    assert {n for n, _ in rec.calls} == NAMES and all(ok for _, ok in rec.calls), rec.calls
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("what", ["dispatch mode", "function mode", "subclass"])
+def test_fast_path_declines(gpu, monkeypatch, what):
+    """Modes that watch calls and tensor subclasses take the Python path, with its values."""
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from fastmlx_amd import ops
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    announce(f"fast path declines: {what}")
+    w, s, b = _weights((64,), 256, 4, 64, gpu, 1)
+    x = torch.randn(4, 256, generator=torch.Generator().manual_seed(2)).bfloat16().to(gpu)
+    want = ops.quantized_matmul(x, w, s, b)
+    rec = _Recorder(ops._fast)
+    monkeypatch.setattr(ops, "_fast", rec)
+    if what == "subclass":
+        got = ops.quantized_matmul(x.as_subclass(_Sub), w, s, b)
+    else:
+        with Dispatch() if what == "dispatch mode" else Function():
+            got = ops.quantized_matmul(x, w, s, b)
+    assert rec.calls == [("quantized_matmul", False)] and torch.equal(got, want)
+
+
+def test_fast_path_raises_the_librarys_refusal(gpu, monkeypatch):
+    """A refused call is made once: the error comes from the C++ path, in the Python path's
+    form, without a second attempt."""
+    from fastmlx_amd import FmxqError, ops
+
+    announce("fast path raises a refusal")
+    w, s, b = _weights((64,), 256, 4, 64, gpu, 1)
+    x = torch.zeros(256 + 8, dtype=torch.bfloat16, device=gpu)[1:257].view(1, 256)
+
+    def second(*_):
+        raise AssertionError("a second attempt")
+
+    fast = ops._fast
+    monkeypatch.setattr(ops, "_fast", None)
+    with pytest.raises(FmxqError) as want:
+        ops.quantized_matmul(x, w, s, b)
+    monkeypatch.setattr(ops, "_fast", fast)
+    monkeypatch.setattr(ops, "load", second)
+    with pytest.raises(FmxqError) as got:
+        ops.quantized_matmul(x, w, s, b)
+    assert str(got.value) == str(want.value) and got.value.code == want.value.code
