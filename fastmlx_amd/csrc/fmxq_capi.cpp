@@ -3,10 +3,11 @@
 // Validation happens here, before anything is enqueued: a failing call returns a
 // nonzero fmxq_status with a message and leaves the stream untouched, the
 // contract mlxgo relies on when it frees the result handle on rc != 0
-// (mlxgo/binding_cgo.go:636-643).  Dispatch by M:
-//   M <= 8 (x rows fit in registers) -> decode GEMV (fmxq_qmv.hip), no MFMA
-//   M <= 32                          -> MFMA GEMV (fmxq_skinny.hip)
-//   otherwise                        -> LDS-dequant MFMA GEMM (fmxq_qmm.hip)
+// (mlxgo/binding_cgo.go:636-643).  quantized_matmul by M (qmm_common has the rules):
+//   few rows           -> decode GEMV (fmxq_qmv.hip), no MFMA
+//   up to 64           -> MFMA walks (fmxq_skinny.hip)
+//   above              -> prefill GEMM (fmxq_qmm_prefill.hip), wide GEMM (fmxq_qmm_wide.hip)
+//   K not a multiple of 64 -> LDS-dequant MFMA GEMM (fmxq_qmm.hip)
 #include <hip/hip_runtime.h>
 
 #include <cstdarg>
@@ -336,7 +337,7 @@ int qmm_common(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
   }
   // qmvw, x shared through LDS and K split over blocks.  int4 group 64 at
   // 9 <= M <= 64, at M <= 16 only for wide outputs or long rows, where it beats
-  // qmvs.  int8 group 64 (dequantizing walk) from M = 9 on every shape, and from
+  // qmvs.  int8 (in groups of 64 dequantizing) from M = 9 on every shape, and from
   // M = 2 / 3 / 8 on long rows / wide / 4096-row outputs, where it beats the dot2
   // GEMV (us, dot2 -> walk: 4096x14336 M = 2 21.1 -> 17.1, M = 5 33.4 -> 17.6;
   // 14336x4096 M = 3 21.0 -> 18.2, M = 5 24.4 -> 18.5 (M = 2 15.4 against 18.1

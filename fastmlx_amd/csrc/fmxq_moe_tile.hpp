@@ -378,13 +378,12 @@ __device__ __forceinline__ void tile_walk(const TileWave<BITS, GS>& tw, uint8_t*
   __builtin_amdgcn_sched_barrier(0);
   issue_w(0);
   __builtin_amdgcn_sched_barrier(0);
-  int k = 0;
+  // K is a multiple of 256 (moe_qmvs_supported), two steps.
 #pragma clang loop unroll(disable)
-  for (; k + 1 < tw.steps; k += 2) {
+  for (int k = 0; k < tw.steps; k += 2) {
     step(std::integral_constant<int, 0>{}, k);
     step(std::integral_constant<int, 1>{}, k + 1);
   }
-  if (k < tw.steps) step(std::integral_constant<int, 0>{}, k);
 }
 
 template <int RT, int NMAT, int BITS, int GS>

@@ -130,6 +130,9 @@ __global__ __launch_bounds__(WAVES * 64, 1) void qmm_wide_kernel(WideArgs wa) {
   // loaded for the next four.
   constexpr int SW = 128 / GS;
   static_assert(SW == 1 || SW == 2 || SW == 4, "group size");
+  // In groups of 32 a lane half has its own group, which the exchange between halves for
+  // two row groups (scale_bias, JT == 2) would give to the other half.
+  static_assert(JT == 1 || GS != 32, "groups of 32 take one row group per wave");
   uint32_t sbA[2 * SW], sbB[2 * SW];
 
   // Work items of this block: dp whole tiles (dealt to the XCDs so that each

@@ -26,7 +26,7 @@
 //   instruction spanning 32 rows at 32 bytes each) runs at under half the HBM
 //   rate of these whole-segment loads.
 //
-// qmv_mfma_kernel (every other int4/int8 case):
+// qmv_mfma_kernel (int4 and int8 where neither walk's limits hold):
 //   v_mfma_f32_32x32x16_bf16 with the weights straight from registers, no LDS:
 //   - lane l holds output column n = l % 32 and, for each 16-byte load, 32 int4
 //     (16 int8) values of row n; lane halves g = l / 32 cover the two halves of a
@@ -39,8 +39,9 @@
 //     (rows >= M read a valid row; their outputs are discarded).
 // In both the K axis is split over the KS waves of a block, which meet in LDS.
 //
-// qmvw_kernel (int4, group 64, 9 <= M <= 64 where it wins: M > 16, or wide
-// outputs / long rows at M <= 16):
+// qmvw_kernel (fmxq_qmvw.hpp; up to 64 rows where it wins: int4 in groups of 64 from 17
+// rows, or from 9 for wide outputs or long rows, in groups of 32 and 128 from 5; int8
+// from 9 rows, on long or wide shapes from 2 to 8):
 //   - the same 16x16x32 tile walk, but the WV waves of a block (4; 8 for 64-row
 //     x tiles on the pipelined walk) own WV W tiles side by side over one K part
 //     and share the block's x rows, which the block
