@@ -321,19 +321,22 @@ int qmm_common(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
     int cus = 0;
     if (int rc = device_cus(&cus)) return rc;
     const fmxq::WidePlan wp = fmxq::qmm_wide_plan(M, N, K, cus);
-    uint32_t* flag = nullptr;
-    bool captured = false;
-    int rc = FMXQ_OK;
-    if (wp.sk_len > 0) {
-      float* unused = nullptr;
-      rc = prefill_workspace(s, wp.ws_floats, &a.ws, &captured);
-      if (!rc) rc = split_workspace(s, fmxq::QmmPlan{2, 0, wp.tiles}, &unused, &a.tile_count, &captured);
-      if (!rc) rc = device_flag(s, &flag);
+    if (!others || fmxq::qmm_wide_pays(a, wp, cus)) {
+      uint32_t* flag = nullptr;
+      bool captured = false;
+      int rc = FMXQ_OK;
+      if (wp.sk_len > 0) {
+        float* unused = nullptr;
+        rc = prefill_workspace(s, wp.ws_floats, &a.ws, &captured);
+        if (!rc)
+          rc = split_workspace(s, fmxq::QmmPlan{2, 0, wp.tiles}, &unused, &a.tile_count, &captured);
+        if (!rc) rc = device_flag(s, &flag);
+      }
+      if (!rc) return hip_status(fmxq::launch_qmm_wide(a, wp, flag, s), op);
+      if (!captured || !others) return rc;
+      a.ws = nullptr;
+      a.tile_count = nullptr;
     }
-    if (!rc) return hip_status(fmxq::launch_qmm_wide(a, wp, flag, s), op);
-    if (!captured || !others) return rc;
-    a.ws = nullptr;
-    a.tile_count = nullptr;
   }
   // qmvw, x shared through LDS and K split over blocks.  int4 group 64 at
   // 9 <= M <= 64, at M <= 16 only for wide outputs or long rows, where it beats
@@ -350,7 +353,8 @@ int qmm_common(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
                                                     : M > 4);
   const bool walk8 = bits == 8 && (M >= 9 || (M >= 2 && K >= 8192) || (M >= 3 && N >= 8192) ||
                                    (M >= 8 && N >= 4096));
-  if ((walk4 || walk8) && M <= fmxq::kQmvwMaxM && fmxq::qmvw_supported(a)) {
+  if ((walk4 || walk8) && M <= fmxq::kQmvwMaxM && fmxq::qmvw_supported(a) &&
+      (!others || fmxq::qmvw_pays(a))) {
     int cus = 0;
     if (int rc = device_cus(&cus)) return rc;
     const fmxq::QmvwPlan qp = fmxq::qmvw_plan(a, cus);

@@ -114,6 +114,8 @@ struct QmvwPlan {
   int64_t ws_floats;  // fp32 partials when parts > 1
 };
 bool qmvw_supported(const QmmArgs& a);
+// Groups of 32 and 128: whether the walk is quicker than the kernels it took over from.
+bool qmvw_pays(const QmmArgs& a);
 QmvwPlan qmvw_plan(const QmmArgs& a, int cus);
 hipError_t launch_qmvw(const QmmArgs& a, const QmvwPlan& p, hipStream_t stream);
 // Its kernels for groups of 32 and 128 (fmxq_qmvw_fmt.hip).
@@ -145,6 +147,8 @@ struct PrefillPlan {
   int64_t ws_floats;
 };
 PrefillPlan qmm_prefill_plan(const QmmArgs& a, int cus);
+// Its output tiles.
+int64_t qmm_prefill_tiles(const QmmArgs& a);
 hipError_t launch_qmm_prefill(const QmmArgs& a, hipStream_t stream);
 // Wide GEMM (fmxq_qmm_wide.hip): 256 (or 128) x 256 tiles, weights dequantized in
 // registers, stream-K over the tiles that do not fill a whole wave of blocks.
@@ -178,6 +182,9 @@ struct WideArgs {
   uint32_t* err;  // raised (bit 2) when a wait for another block's partial gives up
 };
 WidePlan qmm_wide_plan(int64_t M, int64_t N, int64_t K, int cus);
+// Groups of 32 and 128, which the prefill GEMM takes otherwise: whether the wide GEMM's
+// plan is the quicker one.
+bool qmm_wide_pays(const QmmArgs& a, const WidePlan& p, int cus);
 bool qmm_wide_supported(const QmmArgs& a);
 hipError_t launch_qmm_wide(const QmmArgs& a, const WidePlan& p, uint32_t* err, hipStream_t stream);
 // Grouped form (QmmArgs::g_*): grid = N tiles x max_tiles work-list entries.

@@ -507,9 +507,14 @@ TileShape prefill_tile(const QmmArgs& a) {
 
 }  // namespace
 
+int64_t qmm_prefill_tiles(const QmmArgs& a) {
+  const TileShape ts = prefill_tile(a);
+  return ((a.M + ts.bm - 1) / ts.bm) * ((a.N + ts.bn - 1) / ts.bn);
+}
+
 PrefillPlan qmm_prefill_plan(const QmmArgs& a, int cus) {
   const TileShape ts = prefill_tile(a);
-  const int64_t tiles = ((a.M + ts.bm - 1) / ts.bm) * ((a.N + ts.bn - 1) / ts.bn);
+  const int64_t tiles = qmm_prefill_tiles(a);
   const int64_t nk = a.K / kStepK;
   // Tiles of a part-full last wave (or all tiles, when they do not fill the chip
   // once) are split along K while the parts still fill at most one wave and keep

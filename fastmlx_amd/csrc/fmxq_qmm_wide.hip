@@ -540,6 +540,27 @@ WidePlan qmm_wide_plan(int64_t M, int64_t N, int64_t K, int cus) {
   return p;
 }
 
+// Few tiles: a block that ends a tile adds up the partials of all its pieces, one after
+// the other, where the prefill GEMM's K parts meet in a launch of their own.  Over 543
+// shapes of M 128-2048, N 512-28672, K 512-16384 (prefill against wide, us): below 40
+// tiles the wide GEMM is 0.65-0.97 times as fast on four shapes in five (8 bits, 889 x 512
+// x 14592 33.9 / 52.1; 4 bits, 1034 x 512 x 4608 24.8 / 30.2, 1022 x 768 x 9984 36.4 /
+// 47.7), from 40 on 1.2 times as fast on average (806 x 2816 x 5120, 48 tiles, 61.6 / 41);
+// at 8 bits from 52.  Tiles of at most 1024 values are hardly cut and pay from 16 (860 x
+// 1024 x 1024 in 28 tiles 1.19 times), of at most 768 always.
+// 8 bits, one part-full wave of cut tiles where the prefill GEMM has its own tiles whole in
+// one wave: a step of the wide GEMM costs 1.25 of the other's (128 rows of x; twice that
+// for 256) and the cuts about 8 (405 x 13312 x 15104 257 / 288, 774 x 6144 x 1792 33.3 /
+// 38.6; 447 x 10496 x 10240 1.25 times as fast and kept).
+bool qmm_wide_pays(const QmmArgs& a, const WidePlan& p, int cus) {
+  if (a.K > 768 && p.tiles < (a.K <= 1024 ? 16 : a.bits == 8 ? 52 : 40)) return false;
+  if (a.bits == 8 && p.dp == 0 && p.sk_len < p.nk) {
+    const int64_t pt = qmm_prefill_tiles(a);
+    if (pt <= cus && 2 * pt > cus) return 5 * p.sk_len * (p.bm / 128) + 32 <= 4 * p.nk;
+  }
+  return true;
+}
+
 bool qmm_wide_supported(const QmmArgs& a) {
   return a.M >= 1 && a.N >= 1 && a.K % (4 * kS) == 0 && a.K > 0 && a.ldx % 8 == 0 &&
          // 16-byte output stores of 8 outputs

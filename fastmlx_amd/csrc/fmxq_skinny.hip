@@ -372,6 +372,24 @@ bool qmvw_supported(const QmmArgs& a) {
          al(a.biases, a.group_size == 32 ? 16 : 8);
 }
 
+// Where K is short for the outputs, the K parts that fill the chip hold a step or two and
+// their partials and fixup cost more than the product: from N = 21 K up to 16 rows (K up
+// to 1024), 16 K up to 32 (K up to 1792), and up to 64 rows 10 K for K up to 768, 16384
+// for K up to 2048, and all N for K = 512.  Over 702 shapes (prefill GEMM against walk, us): 46 x 21760 x 512
+// 8.1 / 13.7, 26 x 21248 x 512 7.7 / 11.7, 44 x 25344 x 1792 19.4 / 27.3, 40 x 22272 x 1024
+// 13.7 / 17.6, 12 x 21504 x 512 7.5 / 9.0; on the other side of the lines 1.1 times as fast
+// and more.  Past 32 rows the prefill GEMM also keeps outputs below 1024 on long rows (56
+// x 512 x 13312 16.4 / 19.3).  8 bits at up to 4 rows: the dot2 GEMV keeps outputs below
+// 1024 (2 x 512 x 12544 5.1 / 10.7, 3 x 512 x 9728 6.3 / 9.4) and, in groups of 32 (more
+// registers, two waves a SIMD), K up to 2048 (4 x 17280 x 1024 9.4 / 12.5).
+bool qmvw_pays(const QmmArgs& a) {
+  if (a.bits == 8 && a.M <= 4 && (a.N < 1024 || (a.group_size == 32 && a.K <= 2048))) return false;
+  if (a.M > 32 && (a.K <= 512 || (a.K >= 8192 && a.N < 1024))) return false;
+  if (a.M <= 16) return a.K > 1024 || a.N < 21 * a.K;
+  if (a.M <= 32) return a.K > 1792 || a.N < 16 * a.K;
+  return a.K > 2048 || a.N < (a.K <= 768 ? 10 * a.K : 16384);
+}
+
 // Shapes measured on MI355X (4-bit group 64, M = 16 / 32 / 64; the Llama-3-8B
 // projections): long rows (K >= 8192) split K into 8 pipelined parts; wide
 // outputs (N >= 8192) take 32-row W tiles and 4 up-front parts for x tiles of up

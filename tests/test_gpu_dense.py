@@ -655,3 +655,34 @@ def test_quantized_matmul_nonfinite_rows(gpu, oracle, bits, group, M, N, K):
                              group, bits)
     torch.cuda.synchronize()
     _check_nonfinite(to_np(y), x, w, s, b, bits, group, f"{bits} {group} {M} {N} {K}")
+
+
+@pytest.mark.parametrize("bits,group,M,N,K", [
+    (4, 32, 16, 10752, 512), (4, 32, 16, 10744, 512),    # the walk gives way to the prefill GEMM
+    (4, 128, 24, 12288, 768), (4, 128, 24, 12280, 768),
+    (8, 32, 40, 7680, 768), (8, 128, 40, 7672, 768),
+    (4, 32, 33, 1000, 512), (8, 128, 64, 520, 8192),
+    (8, 32, 4, 1016, 8192), (8, 32, 4, 8192, 2048),      # to the dot2 GEMV
+    (8, 128, 4, 8192, 2048),
+    (4, 32, 384, 512, 1280), (4, 32, 384, 3328, 1280),   # the wide GEMM: few tiles, 39 and 42
+    (8, 128, 384, 4352, 1280), (8, 128, 384, 4608, 1280),  # 51 and 54
+    (4, 128, 900, 512, 1024), (4, 128, 1100, 512, 1024),   # 16 and 18
+    (8, 32, 300, 4096, 512),
+    (8, 32, 520, 5632, 1536),   # cut tiles against whole prefill tiles in one wave
+])
+def test_quantized_matmul_other_groups_route_lines(gpu, oracle, bits, group, M, N, K):
+    """Groups of 32 and 128 on both sides of the lines between the walk, the wide GEMM and
+    the kernels they took over from."""
+    from fastmlx_amd import ops
+
+    rng = np.random.default_rng(M + N + K)
+    w, s, b = make_quant(rng, (N,), K, bits, group)
+    x = make_x(rng, M, K)
+    announce(f"route lines bits={bits} group={group} M={M} N={N} K={K}")
+    y = ops.quantized_matmul(to_dev(x, gpu), to_dev(w, gpu), to_dev(s, gpu), to_dev(b, gpu), True,
+                             group, bits)
+    torch.cuda.synchronize()
+    sel = np.unique(np.concatenate([[0, M - 1], rng.choice(M, size=min(M, 12), replace=False)]))
+    import parity
+
+    parity.check_dense(to_np(y)[sel], parity.DenseRef(x[sel], w, s, b, group, bits))
