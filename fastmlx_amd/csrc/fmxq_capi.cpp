@@ -407,6 +407,27 @@ int qmm_common(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
   return hip_status(fmxq::launch_qmm(a, s), op);
 }
 
+// One launch of a general gather kernel against the sort and the walk (one x row per item,
+// formats other than 4 bits in groups of 64; us, general / walk).  The per-item GEMV takes
+// a time per output row of the batch, the walk more per step of K and less per row:
+//   - unsorted batches of up to 16 items over K below 2048 (the walk without a sort) are even
+//     near 16 K rows (512 experts of 512 x 1792, 2 items 3.5 / 9.7; 64 of 768 x 768, 5 and
+//     12 items 5 / 6 and even; 64 of 3328 x 1536, 2 and 8 items 5 / 6 and even);
+//   - sorted ones near 32768 rows (8 experts of 256 x 512, 64 items 5 / 8; 4 of 512 x 256, 64
+//     and 90 items even and 10 / 8), from K = 1024 near 40960, and where few items share
+//     an expert near 49152, in groups of 32 (twice the scales) near 81920 (512 of 256 x
+//     1024, 90 items 6 / 9; 256 of 768 x 4096 in groups of 32, 64 items 9 / 13);
+//   - sorted indices on few experts in a small product suit the 32-slot MFMA kernel (8 of
+//     256 x 256, 700 items 8 / 12; 8 of 1024 x 768, 256 items 11 / 13), many experts do not
+//     (64 of 768 x 768, 700 items 28 / 16).
+bool gather_general(int64_t batch, int64_t E, int64_t N, int64_t K, int group_size, bool mfma) {
+  const int64_t rows = batch * N;
+  if (batch <= fmxq::kMoeUnsortedMaxSlots) return K < 2048 && rows < 16 * K;
+  if (mfma) return batch >= 16 * E && rows * K <= (int64_t(1) << 28);
+  if (K < 1024) return rows < 32768;
+  return rows < (batch >= 4 * E ? 40960 : group_size == 32 ? 81920 : 49152);
+}
+
 }  // namespace
 
 extern "C" {
@@ -544,8 +565,15 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
   uint32_t* flag = nullptr;
   if (int rc = device_flag(static_cast<hipStream_t>(stream), &flag)) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (Mx == 1 && E <= kSortMaxExperts && fmxq::moe_qmvs_supported(N, K, x_batch, bits, group_size) &&
-      aligned16(scales) && aligned16(biases)) {
+  fmxq::GatherArgs ga{x,      w,     scales,  biases, lhs_indices, rhs_indices, y,
+                      batch,  x_batch, lhs_div, Mx,   N,           K,           E,
+                      group_size, bits, flag};
+  const bool mfma = sorted_indices && batch * Mx >= fmxq::kGroupedMinSlots && fmxq::gather_mfma_supported(ga);
+  const bool others = bits != 4 || group_size != 64;
+  const bool general = others && gather_general(batch, E, N, K, group_size, mfma);
+  if (Mx == 1 && !general && E <= kSortMaxExperts &&
+      fmxq::moe_qmvs_supported(N, K, x_batch, bits, group_size) && aligned16(scales) &&
+      aligned16(biases)) {
     // Items sorted by expert, then one grouped product per expert segment; the
     // sort's order maps each sorted item back to its output row.
     if (batch <= fmxq::kMoeUnsortedMaxSlots) {
@@ -598,15 +626,11 @@ int fmxq_gather_qmm(const uint16_t* x, const uint32_t* w, const uint16_t* scales
       if (max_seg > kMaxSegmentsGrid) continue;
       bool captured = false;
       const int rc = sorted(window, max_seg, &captured);
-      if (!captured || (window == walk && bits == 4 && group_size == 64)) return rc;
+      if (!captured || (window == walk && !others)) return rc;
     }
   }
-  fmxq::GatherArgs a{x,      w,     scales,  biases, lhs_indices, rhs_indices, y,
-                     batch,  x_batch, lhs_div, Mx,   N,           K,           E,
-                     group_size, bits, flag};
-  if (sorted_indices && batch * Mx >= fmxq::kGroupedMinSlots && fmxq::gather_mfma_supported(a))
-    return hip_status(fmxq::launch_gather_mfma(a, s), op);
-  return hip_status(fmxq::launch_gather_qmv(a, s), op);
+  if (mfma) return hip_status(fmxq::launch_gather_mfma(ga, s), op);
+  return hip_status(fmxq::launch_gather_qmv(ga, s), op);
 }
 
 int fmxq_device_error(void* stream) {

@@ -76,7 +76,7 @@ def _gather_case(rng, gpu, bits, group, E, S, xb, N, K):
 
 
 @pytest.mark.parametrize("bits,group,E,S,N", [
-    (4, 32, 8, 40, 64), (8, 64, 4, 500, 64), (4, 128, 4, 4200, 64),
+    (4, 32, 8, 40, 1024), (8, 64, 4, 500, 128), (4, 128, 4, 4200, 64),
 ])
 def test_gather_qmm_first_call_captured(gpu, oracle, bits, group, E, S, N):
     """Formats other than 4 bits in groups of 64: the sort's scratch cannot grow, the

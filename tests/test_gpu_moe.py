@@ -1238,3 +1238,45 @@ def test_gather_qmm_few_items_of_a_large_x(gpu, oracle):
     rows = to_np(x[torch.from_numpy(lhs[sel].astype(np.int64)).to(gpu), 0].contiguous())
     ref = parity.gather_refs(rows, *q, np.arange(100, dtype=np.int32), rhs[sel].astype(np.int32))
     parity.check_dense(to_np(y).reshape(S, N)[sel], ref, what="gather_qmm")
+
+
+@pytest.mark.parametrize("bits,group,E,S,N,K,srt", [
+    (4, 32, 7, 107, 520, 1280, True),     # the sorted walk
+    (4, 32, 7, 80, 512, 1280, False),     # 40960 rows: the walk; one item fewer: per item
+    (4, 32, 7, 79, 512, 1280, False),
+    (8, 64, 40, 96, 512, 1024, False),    # few items an expert: 49152 rows and below
+    (8, 64, 40, 95, 512, 1024, False),
+    (8, 32, 40, 160, 512, 1024, False),   # in groups of 32 81920
+    (8, 32, 40, 159, 512, 1024, False),
+    (4, 128, 5, 64, 512, 512, False),     # short K: 32768
+    (4, 128, 5, 63, 512, 512, False),
+    (4, 32, 5, 16, 512, 512, False),      # without a sort: 16 K rows
+    (4, 32, 5, 15, 512, 512, False),
+    (8, 128, 4, 64, 256, 512, True),      # sorted indices: 16 items an expert on the MFMA kernel
+    (8, 128, 4, 63, 256, 512, True),
+    (8, 128, 4, 1100, 512, 512, True),    # a larger product on the walk
+])
+def test_gather_qmm_formats_route_lines(gpu, oracle, bits, group, E, S, N, K, srt):
+    """Formats other than 4 bits in groups of 64 on both sides of the lines between the
+    general kernels and the walk, with a bad expert id."""
+    from fastmlx_amd import FmxqError, ops
+
+    rng = np.random.default_rng(S + N + K)
+    w, s, b = make_quant(rng, (E, N), K, bits, group)
+    rhs = rng.integers(0, E, size=S).astype(np.uint32)
+    rhs[S // 2] = E + 2
+    if srt:
+        rhs.sort()
+    lhs = rng.integers(0, S, size=S).astype(np.uint32)
+    x = make_x(rng, S, 1, K)
+    dev = lambda t: to_dev(t, gpu)
+    announce(f"gather_qmm lines {bits}-bit group {group} E={E} S={S} N={N} K={K} sorted={srt}")
+    y = ops.gather_qmm(dev(x), dev(w), dev(s), dev(b), dev(rhs), dev(lhs), 1, True, group, bits, srt)
+    torch.cuda.synchronize()
+    with pytest.raises(FmxqError):
+        ops.device_error()
+    got, ok = to_np(y).reshape(S, N), rhs < E
+    assert np.all(got[~ok] == 0)
+    ref = parity.gather_refs(x.reshape(S, K), w, s, b, lhs[ok].astype(np.int32),
+                             rhs[ok].astype(np.int32), group, bits)
+    parity.check_dense(got[ok], ref, what="gather_qmm")
