@@ -675,6 +675,16 @@ int gather_dispatch(const fmxq::GatherArgs& a, bool sorted, hipStream_t s) {
 
 namespace {
 
+// A few slots over widths below 2048, in the formats other than 4 bits in groups of 64: the
+// walk without a sort has too few waves for its chain of steps, and the general kernels'
+// four launches end first, in groups of 32 up to 6 slots and in the others up to 3 (time
+// against the walk's: 16 experts, D 1536, I 1792, 4 bits, one slot 0.57 in groups of 32 and
+// 0.72 of 128, 4 slots 0.79 and even; D 1024, I 512, 8 bits in groups of 32 0.7 at one slot
+// and 0.95 at 8).  Widths of 256 and 512 have one or two steps and keep the walk.
+bool glu_general(int64_t S, int64_t D, int64_t I, int group_size, bool others) {
+  return others && S <= (group_size == 32 ? 6 : 3) && D < 2048 && I < 2048 && D + I >= 1024;
+}
+
 int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_gate,
                     const uint16_t* s_gate, const uint16_t* b_gate, const uint32_t* w_up,
                     const uint16_t* s_up, const uint16_t* b_up, const uint32_t* w_down,
@@ -708,7 +718,8 @@ int switch_glu_impl(const uint16_t* x, const uint32_t* inds, const uint32_t* w_g
   // needs less than the tiles, then (formats other than 4 bits in groups of 64) the
   // general kernels below.
   const bool others = bits != 4 || group_size != 64;
-  if (E <= kSortMaxExperts && fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
+  if (E <= kSortMaxExperts && !glu_general(S, D, I, group_size, others) &&
+      fmxq::moe_qmvs_supported(I, D, T, bits, group_size) &&
       fmxq::moe_qmvs_supported(D, I, S + T, bits, group_size) && aligned16(s_gate) &&
       aligned16(b_gate) && aligned16(s_up) && aligned16(b_up) && aligned16(s_down) &&
       aligned16(b_down)) {
@@ -877,7 +888,10 @@ extern "C" int fmxq_switch_glu_combine(
   hipStream_t s = static_cast<hipStream_t>(stream);
   // Decode-sized batches, and batches whose slots rarely share an expert: gate and
   // up into h (no sort), then one kernel for the down projection and the combine.
+  // (One or two slots in groups of 32 over D below 2048: as in glu_general, 0.81 to 0.97
+  // times as long in the calls below.)
   if (fmxq::moe_combine_unsorted(S, E) &&
+      !(S <= 2 && group_size == 32 && glu_general(S, D, I, group_size, true)) &&
       fmxq::moe_down_combine_supported(T, topk, D, I, bits, group_size) &&
       fmxq::moe_qmvs_supported(I, D, T, bits, group_size) && aligned16(s_gate) &&
       aligned16(b_gate) && aligned16(s_up) && aligned16(b_up)) {

@@ -1280,3 +1280,30 @@ def test_gather_qmm_formats_route_lines(gpu, oracle, bits, group, E, S, N, K, sr
     ref = parity.gather_refs(x.reshape(S, K), w, s, b, lhs[ok].astype(np.int32),
                              rhs[ok].astype(np.int32), group, bits)
     parity.check_dense(got[ok], ref, what="gather_qmm")
+
+
+@pytest.mark.parametrize("bits,group", [(4, 32), (4, 128), (8, 64), (8, 32)])
+@pytest.mark.parametrize("T,k", [(1, 1), (1, 2), (1, 3), (2, 2), (3, 2), (7, 1)])
+def test_switch_glu_few_slots_formats(gpu, oracle, bits, group, T, k):
+    """Formats other than 4 bits in groups of 64 at few slots and D, I below 2048: both sides
+    of the lines between the general kernels and the walk, alone and with the combine."""
+    from fastmlx_amd import ops
+
+    rng = np.random.default_rng(bits + group + T * k)
+    E, D, I = 9, 768, 512
+    gate, up, down = _stack(rng, E, D, I, bits, group)
+    x = make_x(rng, T, D)
+    inds = topk_uniform(rng, T, E, k)
+    w16 = oracle.f32_to_bf16(rng.dirichlet(np.ones(k), size=T).astype(np.float32))
+    dev = lambda t: to_dev(t, gpu)
+    stacks = [tuple(map(dev, m)) for m in (gate, up, down)]
+    dx, di = dev(x), dev(inds.astype(np.uint32))
+    announce(f"switch_glu few slots {bits}-bit group {group} T={T} k={k}")
+    y = ops.switch_glu(dx, di, *stacks, group, bits)
+    c = ops.switch_glu_combine(dx, di, *stacks, dev(w16), None, None, group, bits)
+    torch.cuda.synchronize()
+    sref = parity.SwitchRef(x, inds, gate, up, down, group, bits, fused=False)
+    parity.check_switch(to_np(y), sref, what="switch_glu")
+    near = sref.refs[0]
+    parity.combine_check(to_np(c), near, parity.switch_bound(near, near, sref.hscale), w16,
+                         what="switch_glu_combine")
