@@ -89,6 +89,11 @@ int fmxq_dequantize_rows(const uint32_t* w, const uint16_t* scales, const uint16
  * Some shapes sum partial products in a per-stream workspace, grown on first use.
  * While the stream is being captured into a graph it cannot grow: groups of 32
  * and 128 then run on kernels that fit, groups of 64 are refused.
+ * A row of x holding infinities or NaN, or values near bf16's largest, affects its
+ * own outputs only.  From 17 rows on (4 bits in groups of 32 and 128 from 5, 8 bits
+ * from 9), and for expert runs on the 64-slot tiles, these are the dequantized
+ * product's.  Smaller products sum x (offset + q), where such a row gives NaN or
+ * infinities though its product may be finite.
  * Replaces mlx_quantized_matmul (mlxgo/binding_cgo.go:636-643). */
 int fmxq_quantized_matmul(const uint16_t* x, const uint32_t* w, const uint16_t* scales,
                           const uint16_t* biases, uint16_t* y, int64_t M, int64_t N,
