@@ -961,6 +961,9 @@ extern "C" int fmxq_moe_layer(
   // 4096, top-1 at 16 / 24 / 128 tokens 83 / 78, 91 / 113 (302 MB) and 358 / 563; K = 7168,
   // top-4 at 16 / 24 tokens 341 / 340 and 437 / 506 (528 MB)).
   const int64_t shared_bytes = 3 * D * I * bits / 8;
+  // Batches that the forms below took over from the separate calls go back to those where
+  // the stream is being captured and their scratch would have to grow.
+  const bool others = bits != 4 || group_size != 64;
   if (topk <= 15 && fmxq::moe_combine_unsorted(S, E) && D >= 2048 && D <= 16384 &&
       (T <= 16 || T * shared_bytes <= kMoeSharedInMaxBytes) &&
       fmxq::moe_down_combine_supported(T, topk, D, I, bits, group_size) &&
@@ -972,7 +975,7 @@ extern "C" int fmxq_moe_layer(
     MoeScratch m;
     bool captured = false;
     const int rc = moe_scratch(s, S + T, I, 1, &m, op, 0, ScratchSource(), 0, &captured);
-    if (rc && !captured) return rc;
+    if (rc && !(captured && (others || T > 1))) return rc;
     if (!rc) {
       fmxq::MoeArgs gu{x, nullptr, {w_gate, w_up}, {s_gate, s_up}, {b_gate, b_up}, inds, nullptr,
                        nullptr, m.h, nullptr, S, I, D, E, T, flag, group_size, bits, topk};
@@ -1051,7 +1054,7 @@ extern "C" int fmxq_moe_layer(
       int rc = moe_scratch(s, Sa, I, max_seg, &m, op, 0, ScratchSource(), prep, &captured);
       if (!rc)
         rc = stream_arena(s, align_up((size_t)Sa * D * sizeof(uint16_t)), &rows, op, 1, &captured);
-      if (rc && !captured) return rc;
+      if (rc && !(captured && (others || window == fmxq::kMoeTileRows))) return rc;
       if (!rc) return layer(m, static_cast<uint16_t*>(rows));
     }
   }
